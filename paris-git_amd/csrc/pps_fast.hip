@@ -1112,7 +1112,86 @@ k_bottom_build(LevelK<T> L, int singular, double *__restrict__ M, T *__restrict_
     for (int e = tid; e < nb * nb; e += 1024) Minv[e] = (T)M[e];
 }
 
-// The same inverse in LDS for a coarsest level of nb <= 90 cells (the
+// The same inverse for a coarsest level of nb <= 64 cells (every level plan
+// that can halve down to 64 cells), in registers: lane = column, wavefront w
+// holds rows 4w .. 4w+3.  Per pivot the owner wavefront publishes the scaled
+// pivot row (its entry p the pivot's reciprocal) in one of two LDS rows,
+// every wavefront reads it back after the one barrier, and the pivot column
+// of a wavefront's own rows comes from its lane p (readlane).  The
+// arithmetic is k_bottom_build's.  It is a serial
+// chain of nb pivots, bound by the latency of one (LDS write, barrier, LDS
+// read, divide): 31 us for 64 cells, on the critical path of a small solve.
+// The matrix in LDS with two barriers a pivot (k_bottom_build_lds) took
+// 63 us; every wavefront dividing by itself, 38 us.
+__device__ __forceinline__ double lane_value(double v, int lane) {
+    union { double d; int i[2]; } u;
+    u.d = v;
+    u.i[0] = __builtin_amdgcn_readlane(u.i[0], lane);
+    u.i[1] = __builtin_amdgcn_readlane(u.i[1], lane);
+    return u.d;
+}
+constexpr int kBottomReg = 64;   // most cells of the register form
+template <class T>
+__global__ void __launch_bounds__(1024)
+k_bottom_build_reg(LevelK<T> L, int singular, T *__restrict__ Minv) {
+    __shared__ double rows[2][kBottomReg];
+    const int nb = L.nx * L.ny * L.nz;
+    const int lane = threadIdx.x & 63, r0 = (threadIdx.x >> 6) * 4;
+    auto diag = [&](int c) -> double {
+        const int i = c % L.nx, j = (c / L.nx) % L.ny, k = c / (L.nx * L.ny);
+        return singular ? (double)diag_of<T, true>(L, i, j, k, c) : (double)L.dg[c];
+    };
+    const double dsum = lane_value(wsum(lane < nb ? diag(lane) : 0.0), 0);
+    const double alpha = singular ? dsum / ((double)nb * (double)nb) : 0.0;
+    double m[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int c = r0 + q;
+        m[q] = 0.0;
+        if (c >= nb) continue;
+        const int i = c % L.nx, j = (c / L.nx) % L.ny, k = c / (L.nx * L.ny);
+        const int sy = L.nx, sz = L.nx * L.ny;
+        const int xp = c + wrap_p(i, L.nx) - i, xm = c + wrap_m(i, L.nx) - i;
+        const int yp = c + (wrap_p(j, L.ny) - j) * sy, ym = c + (wrap_m(j, L.ny) - j) * sy;
+        const int zp = c + (wrap_p(k, L.nz) - k) * sz, zm = c + (wrap_m(k, L.nz) - k) * sz;
+        double v = lane == c ? diag(c) : 0.0;
+        v -= lane == xp ? (double)L.cx[c] : 0.0;
+        v -= lane == xm ? (double)L.cx[xm] : 0.0;
+        v -= lane == yp ? (double)L.cy[c] : 0.0;
+        v -= lane == ym ? (double)L.cy[ym] : 0.0;
+        v -= lane == zp ? (double)L.cz[c] : 0.0;
+        v -= lane == zm ? (double)L.cz[zm] : 0.0;
+        m[q] = v + alpha;
+    }
+    // the pivot row in buffer p & 1 was last read at pivot p - 2, before the
+    // barrier of pivot p - 1
+    for (int p4 = 0; p4 < nb; p4 += 4) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int p = p4 + u;
+            if (p >= nb) break;
+            double *row = rows[u & 1];
+            if (r0 == p4) {
+                const double piv = 1.0 / lane_value(m[u], p);
+                row[lane] = lane == p ? piv : m[u] * piv;
+            }
+            __syncthreads();
+            const double rc = row[lane];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const double f = lane_value(m[q], p);
+                if (r0 + q == p) m[q] = rc;
+                else if (lane == p) m[q] = -f * rc;
+                else m[q] -= f * rc;
+            }
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+        if (r0 + q < nb && lane < nb) Minv[(r0 + q) * nb + lane] = (T)m[q];
+}
+
+// The same inverse in LDS for a coarsest level of 65 to 90 cells (the
 // matrix and copies of the pivot row and column fit 64 KB): per pivot, the
 // pivot row and column are copied, then every entry is updated from the
 // copies (the arithmetic of k_bottom_build), two barriers per pivot.
@@ -2485,7 +2564,9 @@ static void hier_build(Hier<T> &H, int singular, hipStream_t s) {
         }
     }
     const size_t lds = sizeof(double) * ((size_t)H.nb * H.nb + 2 * (size_t)H.nb);
-    if (lds <= 65536)
+    if (H.nb <= kBottomReg)
+        k_bottom_build_reg<T><<<1, 1024, 0, s>>>(H.lv.back().k(), singular, H.minv.template as<T>());
+    else if (lds <= 65536)
         k_bottom_build_lds<T><<<1, 1024, lds, s>>>(H.lv.back().k(), singular, H.minv.template as<T>());
     else
         k_bottom_build<T><<<1, 1024, 0, s>>>(H.lv.back().k(), singular, H.work.template as<double>(),
