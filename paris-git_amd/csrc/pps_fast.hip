@@ -23,6 +23,7 @@
 // Precision.  PPS_MG_FP64: everything FP64.  PPS_MG_MIXED: the V-cycle
 // runs on FP32 copies of the operator with FP32 vectors and accumulation;
 // the outer CG (residual, update, dot products, mean projection) is FP64.
+#include <algorithm>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
@@ -33,28 +34,12 @@
 #include "pps_internal.h"
 
 #include <hip/hip_ext.h>
+#include "pps_level.h"
 #include "pps_row.h"
+#include "pps_tail.h"
 #include "pps_xcd.h"
 
 namespace pps {
-
-// ---------------------------------------------------------------------
-// kernel-side level view
-// ---------------------------------------------------------------------
-template <class T> struct LevelK {
-    int nx, ny, nz;
-    const T *cx, *cy, *cz, *dg;
-};
-
-// sum over the 64 lanes of a wavefront (result in lane 0)
-__device__ __forceinline__ double wsum(double v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
-    return v;
-}
-
-__device__ __forceinline__ int wrap_m(int i, int n) { return i == 0 ? n - 1 : i - 1; }
-__device__ __forceinline__ int wrap_p(int i, int n) { return i == n - 1 ? 0 : i + 1; }
 
 // Apply the stencil: returns b + sum coupling * neighbour  (the numerator
 // of a Gauss-Seidel update) for cell (i,j,k).
@@ -72,14 +57,6 @@ __device__ __forceinline__ T nb_sum(const LevelK<T> &L, const V *__restrict__ x,
     s += L.cy[cym] * (T)x[cym] + L.cy[c] * (T)x[cyp];
     s += L.cz[czm] * (T)x[czm] + L.cz[c] * (T)x[czp];
     return s;
-}
-
-// Diagonal of a row whose excess A7 - sum(couplings) is zero (every row
-// of a singular system): the sum of its six couplings, in one fixed order
-// shared by every kernel of the V-cycle.
-template <class T>
-__device__ __forceinline__ T diag_sum(T cxm, T cx, T cym, T cy, T czm, T cz) {
-    return ((cxm + cx) + (cym + cy)) + (czm + cz);
 }
 
 // Diagonal of cell c: stored (DGI false) or the coupling sum (DGI true).
@@ -176,38 +153,11 @@ k_rb(LevelK<T> L, const B *__restrict__ b, T *__restrict__ x, int colour) {
 // R[2][rb][np] (first colour new), and under LOP two static buffers of
 // 3 rb + 1 coupling rows.
 // ---------------------------------------------------------------------
-template <int I> struct Ic { static constexpr int value = I; };
-
 // values per LDS coupling buffer of the LOP sweep (2 x 50 KiB), and its
 // threads per workgroup (3 wavefronts per SIMD leave 168 VGPRs a thread;
 // 1024 threads leave 128, and the LOP form spills there)
 constexpr int kLopCap = 12800;
 constexpr int kLopThreads = 768;
-
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
-// Writes the block sum of v to part[block linear id].  Any block of at most
-// 1024 threads whose x extent is a multiple of 64 (each wavefront is 64
-// consecutive linear thread ids); wavefront sums are added in a fixed order.
-__device__ __forceinline__ void block_partial(double v, double *part) {
-    __shared__ double sm[16];
-    const int t = threadIdx.x + blockDim.x * (threadIdx.y + blockDim.y * threadIdx.z);
-    const int b = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
-    const int nw = (blockDim.x * blockDim.y * blockDim.z) >> 6;
-    v = wsum(v);
-    if ((t & 63) == 0) sm[t >> 6] = v;
-    __syncthreads();
-    if (t == 0) {
-        double a = 0.0;
-        for (int w = 0; w < nw; ++w) a += sm[w];
-        part[b] = a;
-    }
-    __syncthreads();
-}
 
 template <class T> struct PairOp {   // operator of one pair at one plane
     T cxa, cxb, cxw;                  // +x couplings of 2m, 2m+1; of 2m-1
@@ -697,11 +647,6 @@ k_prolong_add(int fx, int fy, int fz, T *__restrict__ xf, const T *__restrict__ 
 // a single child.  R = P^T / (fx fy fz) with the level's nominal factors
 // for every coarse cell, so the V-cycle stays symmetric.
 // ---------------------------------------------------------------------
-struct Coarsening {
-    int fx, fy, fz;      // 1 or 2 per axis
-    int cnx, cny, cnz;   // coarse sizes, ceil(n / f)
-};
-
 // coarse b = (1 / (fx fy fz)) * the sum of the children's residuals; one
 // thread per coarse cell
 template <class T, class B, bool DGI>
@@ -1274,21 +1219,17 @@ k_bottom_solve(int nb, const T *__restrict__ Minv, const T *__restrict__ b, T *_
 }
 
 // ---------------------------------------------------------------------
-// The coarse end of a V-cycle in one workgroup, in LDS.  Levels 0 .. nl-1
-// of the tail (level nl-1 is the coarsest, solved with the dense inverse)
-// are staged into LDS at the start: their operators, the right-hand side
-// of level 0 and the inverse.  Colour passes, restriction, the bottom
-// solve and prolongation then run back to back on LDS with workgroup
-// barriers in between, and the iterate of level 0 is written back at the
-// end: one launch instead of several per level, and LDS latency instead of
-// L2 latency per pass.  The arithmetic is that of k_rb / k_resid_restrict /
-// k_bottom_solve / k_prolong_add (in-place colour passes: pre-smoothing
-// colour 0 first, post-smoothing colour 1 first).
+// The coarse end of a V-cycle with trilinear transfers in one workgroup, in
+// LDS (k_tail runs the default transfers).  Levels 0 .. nl-1 of the tail
+// (level nl-1 is the coarsest, solved with the dense inverse) are staged
+// into LDS at the start: their operators, the right-hand side of level 0
+// and the inverse.  The arithmetic is that of k_rb / k_resid_field +
+// k_restrict_tri / k_bottom_solve / k_prolong_tri_add.
 // LDS layout: off[l] = {cx, cy, cz, dg (DGI false only), b, x} of level l,
-// off_minv = the inverse; all offsets in elements of T.
+// off_r the residual of a level, off_minv the inverse; all offsets in
+// elements of T.
 // ---------------------------------------------------------------------
-constexpr int kTailMax = 8;
-template <class T> struct TailK {
+template <class T> struct TailTriK {
     int nl, nb, nu_pre, nu_post;
     LevelK<T> L[kTailMax];   // operators in global memory
     const T *b0;             // right-hand side of level 0 (global)
@@ -1296,15 +1237,13 @@ template <class T> struct TailK {
     const T *minv;
     int off[kTailMax][6];
     int off_minv;
-    int off_r;               // residual of a level (trilinear transfers)
-    int px, py, pz;          // periodic axes (trilinear transfers)
+    int off_r;
+    int px, py, pz;          // periodic axes
 };
 
-// TRI: trilinear transfers (k_resid_field + k_restrict_tri, k_prolong_tri_add
-// on LDS) instead of the 8-child average and piecewise-constant prolongation
-template <class T, bool DGI, bool TRI>
+template <class T, bool DGI>
 __global__ void __launch_bounds__(1024)
-k_tail(TailK<T> K) {
+k_tail_tri(TailTriK<T> K) {
     extern __shared__ unsigned char smem_raw[];
     T *sm = reinterpret_cast<T *>(smem_raw);
     const int tid = threadIdx.x;
@@ -1362,21 +1301,6 @@ k_tail(TailK<T> K) {
         L.dg = sm + K.off[l][3];
         return L;
     };
-    // (a, b, c) of linear index e in an na x nb x nc box: shifts and masks
-    // when na and nb are powers of two (every level of a power-of-two grid),
-    // divisions otherwise
-    auto split = [](int e, int na, int nb, int &a, int &b, int &c) {
-        if (((na & (na - 1)) | (nb & (nb - 1))) == 0) {
-            const int la = __builtin_ctz(na), lb = __builtin_ctz(nb);
-            a = e & (na - 1);
-            b = (e >> la) & (nb - 1);
-            c = e >> (la + lb);
-        } else {
-            a = e % na;
-            b = (e / na) % nb;
-            c = e / (na * nb);
-        }
-    };
     auto cpass = [&](int l, int colour, bool first) {
         const LevelK<T> L = lev(l);
         const T *b = sm + K.off[l][4];
@@ -1385,7 +1309,7 @@ k_tail(TailK<T> K) {
         const int total = nxh * L.ny * L.nz;
         for (int e = tid; e < total; e += NT) {
             int ih, j, k;
-            split(e, nxh, L.ny, ih, j, k);
+            split3(e, nxh, L.ny, ih, j, k);
             const int i = 2 * ih + ((j + k + colour) & 1);
             if (i >= L.nx) continue;
             const long long c = i + (long long)L.nx * (j + (long long)L.ny * k);
@@ -1407,47 +1331,30 @@ k_tail(TailK<T> K) {
         const T *x = sm + K.off[l][5];
         const int cxn = L.nx >> 1, cyn = L.ny >> 1, czn = L.nz >> 1;
         T *bc = sm + K.off[l + 1][4];
-        if constexpr (TRI) {
-            T *r = sm + K.off_r;
-            for (int e = tid; e < L.nx * L.ny * L.nz; e += NT) {
-                int i, j, k;
-                split(e, L.nx, L.ny, i, j, k);
-                r[e] = (b[e] + nb_sum(L, x, i, j, k, e)) - diag_of<T, DGI>(L, i, j, k, e) * x[e];
-            }
-            __syncthreads();
-            const T w[4] = {(T)0.25, (T)0.75, (T)0.75, (T)0.25};
-            for (int e = tid; e < cxn * cyn * czn; e += NT) {
-                int I, J, Kz;
-                split(e, cxn, cyn, I, J, Kz);
-                T acc = 0;
-                for (int c3 = 0; c3 < 4; ++c3) {
-                    const int kf = tri_tap(Kz, c3, L.nz, K.pz);
-                    T accy = 0;
-                    for (int b3 = 0; b3 < 4; ++b3) {
-                        const int jf = tri_tap(J, b3, L.ny, K.py);
-                        const T *row = r + L.nx * (jf + L.ny * kf);
-                        T accx = 0;
-                        for (int a = 0; a < 4; ++a) accx += w[a] * row[tri_tap(I, a, L.nx, K.px)];
-                        accy += w[b3] * accx;
-                    }
-                    acc += w[c3] * accy;
-                }
-                bc[e] = acc * (T)0.125;
-            }
-            __syncthreads();
-            continue;
+        T *r = sm + K.off_r;
+        for (int e = tid; e < L.nx * L.ny * L.nz; e += NT) {
+            int i, j, k;
+            split3(e, L.nx, L.ny, i, j, k);
+            r[e] = (b[e] + nb_sum(L, x, i, j, k, e)) - diag_of<T, DGI>(L, i, j, k, e) * x[e];
         }
+        __syncthreads();
+        const T w[4] = {(T)0.25, (T)0.75, (T)0.75, (T)0.25};
         for (int e = tid; e < cxn * cyn * czn; e += NT) {
             int I, J, Kz;
-            split(e, cxn, cyn, I, J, Kz);
+            split3(e, cxn, cyn, I, J, Kz);
             T acc = 0;
-            for (int dk = 0; dk < 2; ++dk)
-                for (int dj = 0; dj < 2; ++dj)
-                    for (int di = 0; di < 2; ++di) {
-                        const int i = 2 * I + di, j = 2 * J + dj, k = 2 * Kz + dk;
-                        const long long c = i + (long long)L.nx * (j + (long long)L.ny * k);
-                        acc += (b[c] + nb_sum(L, x, i, j, k, c)) - diag_of<T, DGI>(L, i, j, k, c) * x[c];
-                    }
+            for (int c3 = 0; c3 < 4; ++c3) {
+                const int kf = tri_tap(Kz, c3, L.nz, K.pz);
+                T accy = 0;
+                for (int b3 = 0; b3 < 4; ++b3) {
+                    const int jf = tri_tap(J, b3, L.ny, K.py);
+                    const T *row = r + L.nx * (jf + L.ny * kf);
+                    T accx = 0;
+                    for (int a = 0; a < 4; ++a) accx += w[a] * row[tri_tap(I, a, L.nx, K.px)];
+                    accy += w[b3] * accx;
+                }
+                acc += w[c3] * accy;
+            }
             bc[e] = acc * (T)0.125;
         }
         __syncthreads();
@@ -1474,26 +1381,22 @@ k_tail(TailK<T> K) {
         const T *xc = sm + K.off[l + 1][5];
         for (int e = tid; e < fx * fy * fz; e += NT) {
             int i, j, k;
-            split(e, fx, fy, i, j, k);
-            if constexpr (TRI) {
-                const int cz = fz >> 1;
-                const int ia[2] = {i >> 1, tri_other(i, cx, K.px)};
-                const int ja[2] = {j >> 1, tri_other(j, cy, K.py)};
-                const int ka[2] = {k >> 1, tri_other(k, cz, K.pz)};
-                const T w[2] = {(T)0.75, (T)0.25};
-                T acc = 0;
-                for (int c3 = 0; c3 < 2; ++c3) {
-                    T accy = 0;
-                    for (int b3 = 0; b3 < 2; ++b3) {
-                        const T *row = xc + cx * (ja[b3] + cy * ka[c3]);
-                        accy += w[b3] * (w[0] * row[ia[0]] + w[1] * row[ia[1]]);
-                    }
-                    acc += w[c3] * accy;
+            split3(e, fx, fy, i, j, k);
+            const int cz = fz >> 1;
+            const int ia[2] = {i >> 1, tri_other(i, cx, K.px)};
+            const int ja[2] = {j >> 1, tri_other(j, cy, K.py)};
+            const int ka[2] = {k >> 1, tri_other(k, cz, K.pz)};
+            const T w[2] = {(T)0.75, (T)0.25};
+            T acc = 0;
+            for (int c3 = 0; c3 < 2; ++c3) {
+                T accy = 0;
+                for (int b3 = 0; b3 < 2; ++b3) {
+                    const T *row = xc + cx * (ja[b3] + cy * ka[c3]);
+                    accy += w[b3] * (w[0] * row[ia[0]] + w[1] * row[ia[1]]);
                 }
-                xf[e] += acc;
-            } else {
-                xf[e] += xc[(i >> 1) + cx * ((j >> 1) + cy * (k >> 1))];
+                acc += w[c3] * accy;
             }
+            xf[e] += acc;
         }
         __syncthreads();
         for (int q = 0; q < K.nu_post; ++q) {
@@ -2631,8 +2534,9 @@ struct SweepShape {
 template <class T>
 static SweepShape sweep_shape1(int nx, int ny, int nz, int max_rows, int planes, int cus, bool dgi,
                                bool lop) {
-    SweepShape sh;
+    SweepShape sh{};
     const int np = nx / 2;
+    if (np == 0) return sh;   // one cell a row: no pairs (rb 0: colour passes)
     sh.px = (sizeof(T) == 4 && dgi && np % 128 == 0) ? 2 : 1;
     // LOP: two pairs a thread (the one-pair form on 128-wide levels, with
     // the couplings staged the same way, ran slower than the register form:
@@ -2683,13 +2587,12 @@ static SweepShape sweep_shape(int nx, int ny, int nz, int max_rows, int planes, 
     return sweep_shape1<T>(nx, ny, nz, max_rows, planes, cus, dgi, false);
 }
 
-// LDS bytes of a tail that starts at level lt (and its offsets in K)
+// LDS bytes of a trilinear tail that starts at level lt (and its offsets in K)
 template <class T>
-static size_t tail_layout(const Hier<T> &H, int lt, bool dgi, bool tri, TailK<T> *K) {
+static size_t tail_tri_layout(const Hier<T> &H, int lt, bool dgi, TailTriK<T> *K) {
     const int nl = (int)H.lv.size();
-    size_t off = 0;
+    size_t off = (size_t)H.lv[lt].n;   // residual of the tail's top level
     if (K) K->off_r = 0;
-    if (tri && lt < nl) off += (size_t)H.lv[lt].n;   // residual of the tail's top level
     for (int l = lt; l < nl; ++l) {
         const size_t n = (size_t)H.lv[l].n;
         int o[6];
@@ -2706,6 +2609,35 @@ static size_t tail_layout(const Hier<T> &H, int lt, bool dgi, bool tri, TailK<T>
     return off * sizeof(T);
 }
 
+// Most pairs of a tail's top level: k_tail holds them in registers, two a
+// thread, and one a thread of every level below.
+constexpr long long kTailPairs = 2 * kTailThreads;
+// LDS bytes of a tail that starts at level lt (and its offsets in K), 0 if
+// its levels have more pairs than the kernel's threads hold.
+template <class T>
+static size_t tail_layout(const Hier<T> &H, int lt, TailK<T> *K) {
+    const int nl = (int)H.lv.size();
+    const bool one = pairs_of(H.lv[lt].nx, H.lv[lt].ny, H.lv[lt].nz) <= kTailThreads;
+    size_t off = 2 * (one ? (size_t)kTailThreads : (size_t)kTailPairs);   // level 0's iterate
+    auto take = [&](size_t n) { const size_t o = off; off += n; return (int)o; };
+    for (int l = lt; l < nl; ++l) {
+        const Level<T> &L = H.lv[l];
+        const long long tot = (long long)((L.nx + 1) / 2) * L.ny * L.nz;
+        if (l + 1 < nl && tot > (l == lt ? kTailPairs : kTailThreads)) return 0;
+        const int x = l > lt ? take(2 * (size_t)tot) : 0;
+        const int op = l > lt && l + 1 < nl ? take((kPairFields + 2) * (size_t)tot) : 0;
+        const int r = l == lt ? take(2 * (size_t)tot) : 0;
+        if (K) {
+            K->off_x[l - lt] = x;
+            K->off_op[l - lt] = op;
+            if (l == lt) K->off_r = r;
+        }
+    }
+    const int b = take((size_t)H.nb), mi = take((size_t)H.nb * H.nb);
+    if (K) { K->off_b = b; K->off_minv = mi; }
+    return off * sizeof(T);
+}
+
 // How a V-cycle runs (from the handle's options and the system):
 //   nu_pre, nu_post  smoothing sweeps;
 //   dgi              every diagonal is the coupling sum (singular systems);
@@ -2718,7 +2650,7 @@ struct Cycle {
     int nu_pre = 2, nu_post = 2;
     bool dgi = false, fused = true;
     bool tri = false;          // trilinear transfers
-    int per[3] = {0, 0, 0};    // periodic axes (trilinear transfers)
+    int per[3] = {0, 0, 0};    // periodic axes
     int rows = 0, planes = 0;
     long long tail_cells = 4096;
     size_t lds_max = 65536;   // LDS bytes one workgroup may use
@@ -2898,19 +2830,27 @@ static int vcycle(Hier<T> &H, const T *fineb, const Cycle &cy, Prof *prof, hipSt
         for (int l = 1; l < nl; ++l) {
             if (H.lv[l].n <= cy.tail_cells) { lt = l; break; }
         }
-        // the tail must fit the workgroup's LDS, and its transfers are the
-        // regular ones
-        auto tail_regular = [&](int from) {
-            for (int l = from; l + 1 < nl; ++l)
-                if (!H.lv[l].reg) return false;
-            return true;
+        // the tail must fit the workgroup's LDS (and its threads), and hold
+        // more than the coarsest level
+        auto fits = [&](int from) {
+            if (nl - from > kTailMax) return false;
+            const size_t lds = cy.tri ? tail_tri_layout(H, from, dgi, (TailTriK<T> *)nullptr)
+                                      : tail_layout(H, from, (TailK<T> *)nullptr);
+            return lds > 0 && lds <= cy.lds_max;
         };
-        while (lt < nl && (nl - lt > kTailMax || !tail_regular(lt) ||
-                           tail_layout(H, lt, dgi, cy.tri, (TailK<T> *)nullptr) > cy.lds_max))
-            ++lt;
+        while (lt < nl && !fits(lt)) ++lt;
+        if (lt == nl - 1) lt = nl;
     }
+    // the coarse operators (built on the side stream) are needed once the
+    // finest level's smoothing and restriction, which only write the coarse
+    // right-hand side, are done
+    auto wait_coarse = [&]() {
+        if (coarse_ready) (void)hipStreamWaitEvent(s, coarse_ready, 0);
+        coarse_ready = nullptr;
+    };
     for (int l = 0; l < (lt < nl ? lt : nl - 1); ++l) {
         Level<T> &L = H.lv[l];
+        Level<T> &C = H.lv[l + 1];
         const T *b = l == 0 ? fineb : L.b;
         if (fused) {
             if (!(l == 0 && first_done)) rb_sweep(L, l, b, 0, true, cy, prof, s);
@@ -2923,7 +2863,6 @@ static int vcycle(Hier<T> &H, const T *fineb, const Cycle &cy, Prof *prof, hipSt
                 rb_pass(L, l, b, 1, false, dgi, prof, s);
             }
         }
-        Level<T> &C = H.lv[l + 1];
         if (cy.tri) {
             // residual into the free iterate buffer, then full weighting
             const TriK t{L.nx, L.ny, L.nz, cy.per[0], cy.per[1], cy.per[2]};
@@ -2941,17 +2880,11 @@ static int vcycle(Hier<T> &H, const T *fineb, const Cycle &cy, Prof *prof, hipSt
             if (dgi) k_resid_restrict<T, T, true><<<cgrid3(C.nx, C.ny, C.nz), kB3, 0, s>>>(L.k(), b, L.x, C.b);
             else k_resid_restrict<T, T, false><<<cgrid3(C.nx, C.ny, C.nz), kB3, 0, s>>>(L.k(), b, L.x, C.b);
         }
-        // the coarse operators (built on the side stream) are needed from
-        // here on: the finest level's smoothing and restriction only wrote
-        // the coarse right-hand side
-        if (l == 0 && coarse_ready) {
-            (void)hipStreamWaitEvent(s, coarse_ready, 0);
-            coarse_ready = nullptr;
-        }
+        wait_coarse();
     }
-    if (coarse_ready) (void)hipStreamWaitEvent(s, coarse_ready, 0);
-    if (lt < nl) {
-        TailK<T> K;
+    wait_coarse();
+    if (lt < nl && cy.tri) {
+        TailTriK<T> K;
         K.nl = nl - lt;
         K.nb = H.nb;
         K.nu_pre = nu_pre;
@@ -2961,13 +2894,32 @@ static int vcycle(Hier<T> &H, const T *fineb, const Cycle &cy, Prof *prof, hipSt
         K.x0 = H.lv[lt].x;
         K.minv = H.minv.template as<T>();
         K.px = cy.per[0]; K.py = cy.per[1]; K.pz = cy.per[2];
-        const size_t lds = tail_layout(H, lt, dgi, cy.tri, &K);
-        if (cy.tri) {
-            if (dgi) k_tail<T, true, true><<<1, 1024, lds, s>>>(K);
-            else k_tail<T, false, true><<<1, 1024, lds, s>>>(K);
+        const size_t lds = tail_tri_layout(H, lt, dgi, &K);
+        if (dgi) k_tail_tri<T, true><<<1, 1024, lds, s>>>(K);
+        else k_tail_tri<T, false><<<1, 1024, lds, s>>>(K);
+    } else if (lt < nl) {
+        TailK<T> K;
+        K.nl = nl - lt;
+        K.nb = H.nb;
+        K.nu_pre = nu_pre;
+        K.nu_post = nu_post;
+        for (int l = lt; l < nl; ++l) {
+            K.L[l - lt] = H.lv[l].k();
+            K.g[l - lt] = H.lv[l].g;
+        }
+        K.b0 = H.lv[lt].b;
+        K.x0 = H.lv[lt].x;
+        K.minv = H.minv.template as<T>();
+        const size_t lds = tail_layout(H, lt, &K);
+        // one pair a thread while the top level has no more pairs than that
+        const int tot = pairs_of(H.lv[lt].nx, H.lv[lt].ny, H.lv[lt].nz);
+        const int nt = std::min(kTailThreads, std::max(256, (tot + 63) & ~63));
+        if (tot <= nt) {
+            if (dgi) k_tail<T, true, 1><<<1, nt, lds, s>>>(K);
+            else k_tail<T, false, 1><<<1, nt, lds, s>>>(K);
         } else {
-            if (dgi) k_tail<T, true, false><<<1, 1024, lds, s>>>(K);
-            else k_tail<T, false, false><<<1, 1024, lds, s>>>(K);
+            if (dgi) k_tail<T, true, 2><<<1, nt, lds, s>>>(K);
+            else k_tail<T, false, 2><<<1, nt, lds, s>>>(K);
         }
     } else {
         Level<T> &Bt = H.lv.back();
@@ -3034,10 +2986,13 @@ static int fast_ensure(pps_handle *h) {
             f->cus = v;
         // the tail kernel may use all of it
         const int mx = (int)f->lds_max;
-        const void *tails[8] = {(const void *)k_tail<float, true, false>, (const void *)k_tail<float, false, false>,
-                                (const void *)k_tail<double, true, false>, (const void *)k_tail<double, false, false>,
-                                (const void *)k_tail<float, true, true>, (const void *)k_tail<float, false, true>,
-                                (const void *)k_tail<double, true, true>, (const void *)k_tail<double, false, true>};
+        const void *tails[] = {
+            (const void *)k_tail<float, true, 1>, (const void *)k_tail<float, false, 1>,
+            (const void *)k_tail<float, true, 2>, (const void *)k_tail<float, false, 2>,
+            (const void *)k_tail<double, true, 1>, (const void *)k_tail<double, false, 1>,
+            (const void *)k_tail<double, true, 2>, (const void *)k_tail<double, false, 2>,
+            (const void *)k_tail_tri<float, true>, (const void *)k_tail_tri<float, false>,
+            (const void *)k_tail_tri<double, true>, (const void *)k_tail_tri<double, false>};
         for (const void *kt : tails) (void)hipFuncSetAttribute(kt, hipFuncAttributeMaxDynamicSharedMemorySize, mx);
         (void)hipGetLastError();
         f->built = 1;

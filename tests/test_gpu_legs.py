@@ -1,0 +1,62 @@
+"""The V-cycle's fused coarse end (k_tail) against the kernels it replaces.
+
+One refinement step from zero is x = V(b): the default cycle must equal, to
+rounding, the cycle that runs colour by colour (SMOOTH_COLOUR_PASSES: k_rb,
+k_resid_restrict(_g), k_prolong_add(_g) and k_bottom_solve) on the same
+hierarchy.  Shapes at the edges of the tail's thread and pair counts, odd
+and short axes, semi-coarsened boxes, periodic axes, and a non-singular
+operator (stored diagonals).  The bounds are rounding of the precision times
+the few hundred operations of a cycle, as the sweeps' own tests take them.
+"""
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+WALLS, PX, PALL = (0,) * 6, (1, 0, 0, 1, 0, 0), (1,) * 6
+TOL = {"fp64": 1e-12, "mixed": 2e-5}
+
+
+def _cycle(pps, g, A, method, **opt):
+    with pps.Solver(g, method=method, outer=pps.OUTER_REFINE, **opt) as s:
+        p = torch.zeros(g.shape_p, dtype=torch.float64, device="cuda")
+        s.solve(A, p, 1e-300, 1.2, 1)
+    return g.interior(p).clone()
+
+
+def _compare(pps, shape, bc, method, shift=0.0, lengths=(1.0, 1.0, 1.0)):
+    print("cycle vs colour passes", shape, bc, method, shift, lengths, flush=True)
+    g = pps.Grid.make(*shape, bdry_cond=bc, lengths=lengths)
+    rho, u, v, w = pps.synth_fields(g, [(0.4, 0.5, 0.5, 0.2), (0.8, 0.3, 0.6, 0.12)], 1.0, 100.0, 1.5, seed=4)
+    um, vm, wm = pps.pressure_masks(g)
+    A = pps.setup_poisson(g, u, v, w, um, vm, wm, rho, 1.0)
+    pps.remove_rhs_mean(g, A)
+    if shift:
+        A[6] *= 1.0 + shift
+    x = _cycle(pps, g, A, method)
+    ref = _cycle(pps, g, A, method, smoother=pps.SMOOTH_COLOUR_PASSES, tail_cells=-1)
+    err = float((x - ref).abs().max() / ref.abs().max())
+    print(f"   err {err:.2e}", flush=True)
+    assert err <= TOL[method]
+
+
+@pytest.mark.parametrize("method", ["fp64", "mixed"])
+@pytest.mark.parametrize("shape,bc,lengths", [
+    ((32, 32, 32), WALLS, (1.0, 1.0, 1.0)),    # two pairs a thread
+    ((28, 14, 12), PX, (1.0, 1.0, 1.0)),       # 7 wide below: a periodic axis odd, the coarsest
+    ((17, 16, 16), WALLS, (1.0, 1.0, 1.0)),    # missing second cells
+    ((9, 30, 15), WALLS, (1.0, 1.0, 1.0)),
+    ((3, 50, 41), WALLS, (0.06, 1.0, 0.8)),    # one pair a row and a half
+    ((40, 20, 24), PALL, (1.0, 1.0, 1.0)),
+    ((32, 32, 16), WALLS, (1.0, 1.0, 4.0)),    # z kept for two levels
+    ((48, 12, 40), PX, (1.0, 1.0, 1.0)),
+])
+def test_coarse_end_matches_colour_passes(pps, shape, bc, lengths, method):
+    _compare(pps, shape, bc, method, lengths=lengths)
+
+
+@pytest.mark.parametrize("method", ["fp64", "mixed"])
+@pytest.mark.parametrize("shape", [(32, 32, 32), (17, 22, 27)])
+def test_coarse_end_with_stored_diagonals(pps, shape, method):
+    _compare(pps, shape, WALLS, method, shift=0.02)
