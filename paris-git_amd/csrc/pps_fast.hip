@@ -34,6 +34,7 @@
 #include "pps_internal.h"
 
 #include <hip/hip_ext.h>
+#include "pps_leg.h"
 #include "pps_level.h"
 #include "pps_row.h"
 #include "pps_tail.h"
@@ -2797,17 +2798,80 @@ static void rb_sweep(Level<T> &L, int l, const T *b, int c1, bool first, const C
     L.xt = t;
 }
 
-// The finest level's first pre-sweep of a V-cycle on its own, queued ahead
-// by the outer iteration; it returns at once when *skip is non-zero.
+// Whether level l's smoothing legs run as one launch each (k_leg_pre,
+// k_leg_post): the default cycle, on levels small enough that the sweeps'
+// launches cost more than the cells that the legs compute several times
+// over.  FP32: 64^3 9.1 + 9.3 us against 17.4 + 14.6 for the sweeps, 100^3
+// 34 + 51 against 32 + 27.  FP64: 32^3 8.3 + 7.5 us against 16.5 + 10.6, 64^3
+// 17.5 + 19.8 against 29 + 19.
+template <class T> constexpr long long kLegCells = sizeof(T) == 4 ? 300000 : 150000;
 template <class T>
-static void queue_first_sweep(Hier<T> &H, const T *fineb, const Cycle &cy, hipStream_t s, const double *skip) {
-    rb_sweep<T>(H.lv[0], 0, fineb, 0, true, cy, nullptr, s, nullptr, nullptr, skip);
+static bool leg_ok(const Level<T> &L, const Cycle &cy) {
+    return cy.fused && !cy.tri && cy.nu_pre == 2 && cy.nu_post == 2 && cy.rows == 0 && cy.planes == 0 &&
+           L.n <= kLegCells<T>;
 }
-// Whether the look-ahead applies: the finest level runs fused sweeps (one
-// kernel per sweep) and the cycle has a level below it.
+// Planes of a leg's region (its outputs take 8 fewer): 16, or in FP32, whose
+// registers hold three pairs a thread, 24 where that still gives every CU a
+// block.
+template <class T>
+static int leg_ez(const Level<T> &L, const Cycle &cy) {
+    const long long cols = (long long)((L.nx + kLegOut - 1) / kLegOut) * ((L.ny + kLegOut - 1) / kLegOut);
+    return sizeof(T) == 4 && cols * ((L.nz + 15) / 16) >= cy.cus ? 24 : 16;
+}
+template <class T>
+static LegK leg_grid(const Level<T> &L, int ez, const Cycle &cy) {
+    const int oz = ez - 2 * kLegHalo;
+    return LegK{cy.per[0], cy.per[1], cy.per[2], (L.nx + kLegOut - 1) / kLegOut, (L.ny + kLegOut - 1) / kLegOut,
+                (L.nz + oz - 1) / oz};
+}
+template <class T>
+static void leg_pre(const Level<T> &L, const Level<T> &C, const T *b, const Cycle &cy, hipStream_t s,
+                    const double *skip = nullptr) {
+    const int ez = leg_ez(L, cy);
+    const LegK g = leg_grid(L, ez, cy);
+    auto k = cy.dgi ? k_leg_pre<T, true, 16> : k_leg_pre<T, false, 16>;
+    if constexpr (sizeof(T) == 4)
+        if (ez == 24) k = cy.dgi ? k_leg_pre<T, true, 24> : k_leg_pre<T, false, 24>;
+    k<<<g.tx * g.ty * g.tz, kLegThreads, 0, s>>>(L.k(), g, L.g, b, L.x, C.b, skip);
+}
+// dot: block partials, as rb_sweep's (returns their block count)
+template <class T>
+static int leg_post(Level<T> &L, int l, const Level<T> &C, const T *b, const Cycle &cy, Prof *prof, hipStream_t s,
+                    double *dot) {
+    const int ez = leg_ez(L, cy);
+    const LegK g = leg_grid(L, ez, cy);
+    const int blocks = g.tx * g.ty * g.tz;
+    auto k = dot ? (cy.dgi ? k_leg_post<T, true, 16, true> : k_leg_post<T, false, 16, true>)
+                 : (cy.dgi ? k_leg_post<T, true, 16, false> : k_leg_post<T, false, 16, false>);
+    if constexpr (sizeof(T) == 4)
+        if (ez == 24)
+            k = dot ? (cy.dgi ? k_leg_post<T, true, 24, true> : k_leg_post<T, false, 24, true>)
+                    : (cy.dgi ? k_leg_post<T, true, 24, false> : k_leg_post<T, false, 24, false>);
+    // algorithmic bytes: as a fused sweep's, plus the coarse correction
+    const double bytes = (double)sizeof(T) * ((double)L.n * (cy.dgi ? 6.0 : 7.0) + (double)C.n);
+    hipEvent_t *e = l == 0 && prof ? prof->begin(bytes) : nullptr;
+    if (e)
+        hipExtLaunchKernelGGL(k, dim3(blocks), dim3(kLegThreads), 0, s, e[0], e[1], 0, L.k(), g, L.g, b,
+                              (const T *)L.x, (const T *)C.x, L.xt, dot);
+    else
+        k<<<blocks, kLegThreads, 0, s>>>(L.k(), g, L.g, b, L.x, C.x, L.xt, dot);
+    std::swap(L.x, L.xt);
+    return blocks;
+}
+
+// The start of a V-cycle on the finest level, queued ahead by the outer
+// iteration: its pre-leg, or else its first pre-sweep (which swaps the
+// iterate buffers); returns at once when *skip is non-zero.
+template <class T>
+static void queue_first(Hier<T> &H, const T *fineb, const Cycle &cy, hipStream_t s, const double *skip) {
+    if (leg_ok(H.lv[0], cy)) leg_pre(H.lv[0], H.lv[1], fineb, cy, s, skip);
+    else rb_sweep<T>(H.lv[0], 0, fineb, 0, true, cy, nullptr, s, nullptr, nullptr, skip);
+}
+// Whether the look-ahead applies: the finest level runs legs or fused sweeps
+// and the cycle has a level below it.
 template <class T>
 static bool can_queue_first(const Hier<T> &H, const Cycle &cy) {
-    return cy.fused && H.lv.size() > 1 && sweep_fused(H.lv[0], cy);
+    return cy.fused && H.lv.size() > 1 && (leg_ok(H.lv[0], cy) || sweep_fused(H.lv[0], cy));
 }
 
 // one V-cycle: x_0 = V(b_0).  fineb: the fine right-hand side (the FP64
@@ -2815,7 +2879,7 @@ static bool can_queue_first(const Hier<T> &H, const Cycle &cy) {
 // and the last fine sweep is a fused one that can, that sweep writes the
 // block sums of b_0 x_0, x_0 and b_0 there (as k_dot_rz lays them out);
 // returns their block count, 0 if it did not.  first_done: the finest
-// level's first pre-sweep is already queued (queue_first_sweep).
+// level's first pre-sweep or pre-leg is already queued (queue_first).
 template <class T>
 static int vcycle(Hier<T> &H, const T *fineb, const Cycle &cy, Prof *prof, hipStream_t s,
                   double *dot = nullptr, hipEvent_t coarse_ready = nullptr, bool first_done = false) {
@@ -2852,6 +2916,11 @@ static int vcycle(Hier<T> &H, const T *fineb, const Cycle &cy, Prof *prof, hipSt
         Level<T> &L = H.lv[l];
         Level<T> &C = H.lv[l + 1];
         const T *b = l == 0 ? fineb : L.b;
+        if (leg_ok(L, cy)) {
+            if (!(l == 0 && first_done)) leg_pre(L, C, b, cy, s);
+            wait_coarse();
+            continue;
+        }
         if (fused) {
             if (!(l == 0 && first_done)) rb_sweep(L, l, b, 0, true, cy, prof, s);
             for (int q = 1; q < nu_pre; ++q) rb_sweep(L, l, b, 0, false, cy, prof, s);
@@ -2930,6 +2999,12 @@ static int vcycle(Hier<T> &H, const T *fineb, const Cycle &cy, Prof *prof, hipSt
         Level<T> &L = H.lv[l];
         const Level<T> &C = H.lv[l + 1];
         const T *b = l == 0 ? fineb : L.b;
+        if (leg_ok(L, cy)) {
+            double *d = l == 0 ? dot : nullptr;
+            const int blocks = leg_post(L, l, C, b, cy, prof, s, d);
+            if (d) ndot = blocks;
+            continue;
+        }
         // the first fused post-sweep adds a piecewise-constant correction
         // as it loads x; the trilinear one is a pass of its own
         const bool fold = nu_post > 0 && sweep_fused(L, cy) && !cy.tri && L.reg;
@@ -3114,7 +3189,8 @@ static int fast_setup(pps_handle *h, const double *dA, const double *dp, bool mi
             Level<double> &L0 = H.lv[0];
             L0.cx = o64; L0.cy = o64 + n; L0.cz = o64 + 2 * n; L0.dg = o64 + 3 * n;
             L0.b = nullptr;
-            L0.x = V.z;
+            L0.x = V.z;   // the cycle swaps the two iterate buffers
+            L0.xt = H.bufs[0].template as<double>();
             hier_build(H, singular, st);
         }
         return PPS_OK;
@@ -3296,7 +3372,7 @@ static int outer_iterate(pps_handle *h, Hier<T> &H, bool mixed, double tol_abs, 
             k_scal_rr<<<1, 1024, 0, s>>>(part, zg.blocks, 0, S, h->mbox, ++h->mseq, nullptr, N, tol_abs);
         }
         if (ahead && k < maxit) {
-            queue_first_sweep(H, fb, cy, s, S + S_STOP);
+            queue_first(H, fb, cy, s, S + S_STOP);
             queued = true;
         }
         PPS_HIP(hipGetLastError());
@@ -3308,8 +3384,8 @@ static int outer_iterate(pps_handle *h, Hier<T> &H, bool mixed, double tol_abs, 
         if (!(t2 == t2) || t2 > 1e300) { *it = k; return PPS_ERR_DIVERGED; }
         if (stop) {
             // the queued sweep returned without writing: undo its swap of
-            // the finest level's iterate buffers
-            if (queued) std::swap(H.lv[0].x, H.lv[0].xt);
+            // the finest level's iterate buffers (a leg swaps none)
+            if (queued && !leg_ok(H.lv[0], cy)) std::swap(H.lv[0].x, H.lv[0].xt);
             queued = false;
             break;
         }

@@ -1,4 +1,5 @@
-"""The V-cycle's fused coarse end (k_tail) against the kernels it replaces.
+"""The V-cycle's fused smoothing legs (k_leg_pre / k_leg_post) and coarse end
+(k_tail) against the kernels they replace.
 
 One refinement step from zero is x = V(b): the default cycle must equal, to
 rounding, the cycle that runs colour by colour (SMOOTH_COLOUR_PASSES: k_rb,
@@ -60,3 +61,41 @@ def test_coarse_end_matches_colour_passes(pps, shape, bc, lengths, method):
 @pytest.mark.parametrize("shape", [(32, 32, 32), (17, 22, 27)])
 def test_coarse_end_with_stored_diagonals(pps, shape, method):
     _compare(pps, shape, WALLS, method, shift=0.02)
+
+
+@pytest.mark.parametrize("method", ["fp64", "mixed"])
+@pytest.mark.parametrize("shape,bc,lengths", [
+    ((40, 40, 40), WALLS, (1.0, 1.0, 1.0)),    # a finest level of whole tiles
+    ((41, 35, 37), WALLS, (1.0, 1.0, 1.0)),    # remainders in every direction
+    ((64, 23, 50), PX, (1.0, 1.0, 1.0)),
+    ((48, 48, 32), PALL, (1.0, 1.0, 1.0)),
+    ((2, 96, 48), WALLS, (0.02, 1.0, 0.5)),    # one pair a row
+    ((64, 64, 17), WALLS, (1.0, 1.0, 1.5)),    # x, y halved, z kept
+    ((64, 64, 64), WALLS, (1.0, 1.0, 1.0)),    # 24-plane regions in FP32
+])
+def test_legs_match_colour_passes(pps, shape, bc, lengths, method):
+    _compare(pps, shape, bc, method, lengths=lengths)
+
+
+@pytest.mark.parametrize("method", ["fp64", "mixed"])
+def test_legs_with_stored_diagonals(pps, method):
+    _compare(pps, (45, 40, 33), WALLS, method, shift=0.02)
+
+
+def test_repeated_solves_swap_buffers(pps):
+    """An odd number of cycles leaves the finest level's two iterate buffers
+    swapped; a second solve on the handle must not see them as one."""
+    g = pps.Grid.make(40, 44, 36)
+    rho, u, v, w = pps.synth_fields(g, [(0.4, 0.5, 0.5, 0.2)], 1.0, 100.0, 1.5, seed=4)
+    um, vm, wm = pps.pressure_masks(g)
+    A = pps.setup_poisson(g, u, v, w, um, vm, wm, rho, 1.0)
+    pps.remove_rhs_mean(g, A)
+    brms = float(torch.sqrt((A[7] ** 2).mean()))
+    with pps.Solver(g, method="fp64") as s:
+        for its in (1, 2, 3):
+            p = torch.zeros(g.shape_p, dtype=torch.float64, device="cuda")
+            s.solve(A, p, 1e-300, 1.2, its)
+            p.zero_()
+            it, _ = s.solve(A, p, 1e-10 * brms, 1.2, 60, allow_maxit=False)
+            print(f"after {its} cycles: {it} iterations", flush=True)
+            assert it <= 15
