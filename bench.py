@@ -89,7 +89,7 @@ def solve_bytes(n3, iters, S, nu_pre=2, nu_post=2, tail_cells=4096):
     return setup + iters * (v + outer) + final
 
 
-TRAFFIC_FILE = os.path.join(ROOT, "profiles", "k_rb_sweep_drops256_traffic.md")
+TRAFFIC_FILE = os.path.join(ROOT, "profiles", "k_march_drops256_traffic.md")
 
 
 def measured_traffic():
@@ -416,15 +416,16 @@ def main():
     f64 = res["fp64"]
     n_cells = grid.cells
     roof = {
-        "kernel": "k_rb_sweep<float, false, 2, true, true, false, true, false, true> (finest-level "
-                  "fused red-black Gauss-Seidel sweep, FP32, couplings staged through LDS)",
+        "kernel": "k_march<float, false, true, true> (finest-level post-smoothing leg: the coarse "
+                  "correction, two red-black Gauss-Seidel sweeps and the CG dot products in one pass "
+                  "over memory, FP32; bytes counted once for the pass, not once a sweep)",
         "bound": "hbm",
         "achieved": round(m["smoother_GBps"], 1),
         "peak": HBM_PEAK_GBPS,
         "unit": "GB/s",
         "frac": round(m["smoother_GBps"] / HBM_PEAK_GBPS, 4),
         "traffic": measured_traffic(),
-        "traffic_source": ("profiles/k_rb_sweep_drops256_traffic.md: rocprofv3 --pmc FETCH_SIZE and "
+        "traffic_source": ("profiles/k_march_drops256_traffic.md: rocprofv3 --pmc FETCH_SIZE and "
                            "WRITE_SIZE of this kernel in 'bench.py --only mixed --steps 1', calibrated "
                            "by 'bench.py --copy-calib 1024' (not measured in this run)"),
         "launches": m["launches"],

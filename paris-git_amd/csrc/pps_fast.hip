@@ -36,6 +36,7 @@
 #include <hip/hip_ext.h>
 #include "pps_leg.h"
 #include "pps_level.h"
+#include "pps_march.h"
 #include "pps_row.h"
 #include "pps_tail.h"
 #include "pps_xcd.h"
@@ -2859,19 +2860,76 @@ static int leg_post(Level<T> &L, int l, const Level<T> &C, const T *b, const Cyc
     return blocks;
 }
 
+// Whether level l's legs march (k_march): the default cycle on the larger
+// levels of a singular system.  256^3 FP32: 111 + 142 us against 198 + 162
+// for the sweeps and the restriction (FP64 169 + 218 against 484 + 409);
+// 128^3 FP32 23 + 25 against 42 + 38, FP64 39 + 36 against 82 + 54; 100^3
+// FP32 20 + 20 against 32 + 38.  64^3 FP64 16.5 + 18 against 17.5 + 21 for
+// the one-region legs; 64^3 FP32 15 + 13 against their 9.1 + 9.3.
+template <class T>
+static bool march_ok(const Level<T> &L, const Cycle &cy) {
+    return cy.fused && !cy.tri && cy.dgi && cy.nu_pre == 2 && cy.nu_post == 2 && cy.rows == 0 && cy.planes == 0 &&
+           L.n > kLegCells<T> && L.n * (long long)sizeof(T) < (1LL << 32) && L.nx >= 16 && L.ny >= 16 && L.nz >= 8;
+}
+// Blocks of a marching leg: the planes of a block that minimise rounds of
+// blocks (two fit a CU in FP32, one in FP64) x steps of a block.
+template <class T>
+static MarchK march_grid(const Level<T> &L, const Cycle &cy, int *blocks) {
+    MarchK g{cy.per[0], cy.per[1], cy.per[2], (L.nx + kMarchOut - 1) / kMarchOut, (L.ny + kMarchOut - 1) / kMarchOut, 2};
+    const long long cols = (long long)g.tx * g.ty;
+    const int slots = cy.cus * (sizeof(T) == 4 ? 2 : 1);
+    long long best = -1;
+    for (int zc = 2; zc <= ((L.nz + 1) & ~1); zc += 2) {
+        const long long nb = cols * ((L.nz + zc - 1) / zc);
+        const long long cost = ((nb + slots - 1) / slots) * (zc + 2 * kMarchHalo);
+        if (best < 0 || cost < best) { best = cost; g.zc = zc; }
+    }
+    *blocks = (int)(cols * ((L.nz + g.zc - 1) / g.zc));
+    return g;
+}
+template <class T>
+static void march_pre(const Level<T> &L, const Level<T> &C, const T *b, const Cycle &cy, hipStream_t s,
+                      const double *skip = nullptr) {
+    int blocks;
+    const MarchK g = march_grid(L, cy, &blocks);
+    auto k = L.nx % (16 / (int)sizeof(T)) == 0 ? k_march<T, true, false, true> : k_march<T, true, false, false>;
+    k<<<blocks, kMarchThreads, 0, s>>>(L.k(), g, L.g, b, nullptr, nullptr, L.x, C.b, nullptr, skip);
+}
+template <class T>
+static int march_post(Level<T> &L, int l, const Level<T> &C, const T *b, const Cycle &cy, Prof *prof, hipStream_t s,
+                      double *dot) {
+    int blocks;
+    const MarchK g = march_grid(L, cy, &blocks);
+    const bool v16 = L.nx % (16 / (int)sizeof(T)) == 0;
+    auto k = dot ? (v16 ? k_march<T, false, true, true> : k_march<T, false, true, false>)
+                 : (v16 ? k_march<T, false, false, true> : k_march<T, false, false, false>);
+    // algorithmic bytes: 3 couplings, b, half the iterate and the coarse
+    // correction in, the iterate out
+    const double bytes = (double)sizeof(T) * ((double)L.n * 5.5 + (double)C.n);
+    hipEvent_t *e = l == 0 && prof ? prof->begin(bytes) : nullptr;
+    if (e)
+        hipExtLaunchKernelGGL(k, dim3(blocks), dim3(kMarchThreads), 0, s, e[0], e[1], 0, L.k(), g, L.g, b,
+                              (const T *)L.x, (const T *)C.x, L.xt, (T *)nullptr, dot, (const double *)nullptr);
+    else
+        k<<<blocks, kMarchThreads, 0, s>>>(L.k(), g, L.g, b, L.x, C.x, L.xt, nullptr, dot, nullptr);
+    std::swap(L.x, L.xt);
+    return blocks;
+}
+
 // The start of a V-cycle on the finest level, queued ahead by the outer
 // iteration: its pre-leg, or else its first pre-sweep (which swaps the
 // iterate buffers); returns at once when *skip is non-zero.
 template <class T>
 static void queue_first(Hier<T> &H, const T *fineb, const Cycle &cy, hipStream_t s, const double *skip) {
     if (leg_ok(H.lv[0], cy)) leg_pre(H.lv[0], H.lv[1], fineb, cy, s, skip);
+    else if (march_ok(H.lv[0], cy)) march_pre(H.lv[0], H.lv[1], fineb, cy, s, skip);
     else rb_sweep<T>(H.lv[0], 0, fineb, 0, true, cy, nullptr, s, nullptr, nullptr, skip);
 }
 // Whether the look-ahead applies: the finest level runs legs or fused sweeps
 // and the cycle has a level below it.
 template <class T>
 static bool can_queue_first(const Hier<T> &H, const Cycle &cy) {
-    return cy.fused && H.lv.size() > 1 && (leg_ok(H.lv[0], cy) || sweep_fused(H.lv[0], cy));
+    return cy.fused && H.lv.size() > 1 && (leg_ok(H.lv[0], cy) || march_ok(H.lv[0], cy) || sweep_fused(H.lv[0], cy));
 }
 
 // one V-cycle: x_0 = V(b_0).  fineb: the fine right-hand side (the FP64
@@ -2918,6 +2976,11 @@ static int vcycle(Hier<T> &H, const T *fineb, const Cycle &cy, Prof *prof, hipSt
         const T *b = l == 0 ? fineb : L.b;
         if (leg_ok(L, cy)) {
             if (!(l == 0 && first_done)) leg_pre(L, C, b, cy, s);
+            wait_coarse();
+            continue;
+        }
+        if (march_ok(L, cy)) {
+            if (!(l == 0 && first_done)) march_pre(L, C, b, cy, s);
             wait_coarse();
             continue;
         }
@@ -3002,6 +3065,12 @@ static int vcycle(Hier<T> &H, const T *fineb, const Cycle &cy, Prof *prof, hipSt
         if (leg_ok(L, cy)) {
             double *d = l == 0 ? dot : nullptr;
             const int blocks = leg_post(L, l, C, b, cy, prof, s, d);
+            if (d) ndot = blocks;
+            continue;
+        }
+        if (march_ok(L, cy)) {
+            double *d = l == 0 ? dot : nullptr;
+            const int blocks = march_post(L, l, C, b, cy, prof, s, d);
             if (d) ndot = blocks;
             continue;
         }
@@ -3385,7 +3454,7 @@ static int outer_iterate(pps_handle *h, Hier<T> &H, bool mixed, double tol_abs, 
         if (stop) {
             // the queued sweep returned without writing: undo its swap of
             // the finest level's iterate buffers (a leg swaps none)
-            if (queued && !leg_ok(H.lv[0], cy)) std::swap(H.lv[0].x, H.lv[0].xt);
+            if (queued && !leg_ok(H.lv[0], cy) && !march_ok(H.lv[0], cy)) std::swap(H.lv[0].x, H.lv[0].xt);
             queued = false;
             break;
         }

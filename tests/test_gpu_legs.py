@@ -1,5 +1,5 @@
-"""The V-cycle's fused smoothing legs (k_leg_pre / k_leg_post) and coarse end
-(k_tail) against the kernels they replace.
+"""The V-cycle's fused smoothing legs (k_leg_pre / k_leg_post on small levels,
+k_march on large ones) and coarse end (k_tail) against the kernels they replace.
 
 One refinement step from zero is x = V(b): the default cycle must equal, to
 rounding, the cycle that runs colour by colour (SMOOTH_COLOUR_PASSES: k_rb,
@@ -74,6 +74,23 @@ def test_coarse_end_with_stored_diagonals(pps, shape, method):
     ((64, 64, 64), WALLS, (1.0, 1.0, 1.0)),    # 24-plane regions in FP32
 ])
 def test_legs_match_colour_passes(pps, shape, bc, lengths, method):
+    _compare(pps, shape, bc, method, lengths=lengths)
+
+
+@pytest.mark.parametrize("method", ["fp64", "mixed"])
+@pytest.mark.parametrize("shape,bc,lengths", [
+    ((72, 72, 72), WALLS, (1.0, 1.0, 1.0)),    # whole tiles
+    ((73, 67, 71), WALLS, (1.0, 1.0, 1.0)),    # odd rows (4-byte loads), remainders of one tile row
+    ((76, 50, 98), WALLS, (1.0, 1.0, 1.0)),    # a last tile of two columns
+    ((64, 81, 70), PX, (1.0, 1.0, 1.0)),
+    ((66, 70, 76), WALLS, (1.0, 1.0, 1.0)),    # even rows, no multiple of 16 bytes in FP32
+    ((96, 64, 64), PALL, (1.0, 1.0, 1.0)),
+    ((40, 96, 96), WALLS, (2.0, 1.0, 1.0)),    # x kept
+    ((80, 77, 60), WALLS, (1.0, 1.0, 2.0)),    # z kept, y odd
+    ((96, 24, 96), PALL, (1.0, 0.25, 1.0)),    # one tile of rows, wrapped onto itself (FP64)
+    ((128, 150, 16), PX, (1.0, 1.0, 0.1)),     # short columns
+])
+def test_marching_legs_match_colour_passes(pps, shape, bc, lengths, method):
     _compare(pps, shape, bc, method, lengths=lengths)
 
 
