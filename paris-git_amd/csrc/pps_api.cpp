@@ -128,6 +128,8 @@ extern "C" int pps_finalize(pps_handle *h) {
     h->spacing.release();
     h->widths.release();
     h->asplit.release();
+    h->sorold.release();
+    if (h->sorbox) (void)hipHostFree(h->sorbox);
     h->red.release();
     if (h->pinned) (void)hipHostFree(h->pinned);
     if (h->mbox) (void)hipHostFree(h->mbox);

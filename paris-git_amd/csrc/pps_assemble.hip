@@ -203,11 +203,7 @@ double *stats_partials(pps_handle *h) {
     if (ensure_red(h) != PPS_OK) return nullptr;
     return red_part(h);
 }
-int stats_finish(pps_handle *h, int nblocks, int ncomp, int maxmask, double *out, hipStream_t s) {
-    PPS_TRY(red_finish(h, nblocks, ncomp, maxmask, s));
-    for (int c = 0; c < ncomp; ++c) out[c] = h->pinned[c];
-    return PPS_OK;
-}
+int *stats_flag(pps_handle *h) { return red_flag(h) + 8; }
 int fs_residual_stats(pps_handle *h, const Dims &d, const double *A, const double *p,
                       const int *pcmask, int flag, double out[4], hipStream_t s) {
     PPS_TRY(ensure_red(h));

@@ -146,6 +146,14 @@ struct Mailbox {
     unsigned long long seq;
 };
 
+// Totals of one RB-SOR iteration, written by the device into coherent host
+// memory (seq last); a ring of them, one for each iteration in flight.
+struct SorBox {
+    double st[4], bad, stop;
+    unsigned long long seq;
+};
+constexpr int kSorBoxes = 8;
+
 }  // namespace pps
 
 struct pps_handle {
@@ -168,6 +176,9 @@ struct pps_handle {
     pps::DevBuf hmask, hpgas;      // pcmask / P_gas staging for host FreeSolver calls
     pps::DevBuf spacing;           // dx, dxh, x per axis (handle_spacing)
     pps::DevBuf asplit;            // colour-split A of the SOR sweeps (8n doubles)
+    pps::DevBuf sorold;            // the first colour before its last pass (n / 2 doubles)
+    pps::SorBox *sorbox = nullptr; // coherent host memory (first SOR solve)
+    unsigned long long sorseq = 0; // iterations that may have used it
     // row weights of the fast methods (pps_set_cell_widths): wx | wy | wz on
     // the device, normalised to a maximum of 1, and min wx * min wy * min wz
     pps::DevBuf widths;
@@ -240,11 +251,11 @@ int handle_spacing(pps_handle *h, const double *dh[3], hipStream_t s);
 // dst[a] = src[a] on the ghost layers of three padded arrays (interiors
 // untouched).
 int copy_ghosts(const Dims &d, const double *const src[3], double *const dst[3], hipStream_t s);
-// Block partials written by other kernels (comp c of block b at
-// part[c * kRedBlocks + b]), then their fixed-order totals (comps in
-// maxmask take the maximum) into out; synchronises.
+// Block partials written by other kernels: comp c of block b at
+// part[c * kRedBlocks + b].
 double *stats_partials(pps_handle *h);
-int stats_finish(pps_handle *h, int nblocks, int ncomp, int maxmask, double *out, hipStream_t s);
+// a device word beside them (the SOR iterations' stop flag)
+int *stats_flag(pps_handle *h);
 // {sum |r|, sum r^2, max |r|} (calcResiduals before normalisation).
 int fs_residual_stats(pps_handle *h, const Dims &d, const double *A, const double *p,
                       const int *pcmask, int flag, double out[4], hipStream_t s);

@@ -86,27 +86,6 @@ k_split_colours(LvlK L, const double *__restrict__ A, double *__restrict__ As) {
     for (int s = 0; s < 8; ++s) a[s * hn + h] = A[s * n + c];
 }
 
-// k_rb_pass on the colour-split A (the same expression)
-__global__ void __launch_bounds__(256)
-k_rb_pass_split(LvlK L, const double *__restrict__ As, double *__restrict__ p,
-                const int *__restrict__ pcmask, int flag, double beta, int colour) {
-    const int j = blockIdx.y * blockDim.y + threadIdx.y;
-    const int k = blockIdx.z;
-    const int m = blockIdx.x * blockDim.x + threadIdx.x;
-    const int i = 2 * m + ((j + k + colour) & 1);
-    if (j >= L.ny || i >= L.nx) return;
-    const long long q = ipad(L, i, j, k);
-    if (pcmask && !(flag == 1 ? pcmask[q] == 0 : (pcmask[q] == 1 || pcmask[q] == 2))) return;
-    const long long hn = lk_cells(L) / 2;
-    const long long h = ((long long)k * L.ny + j) * (L.nx / 2) + m;
-    const double *a = As + (long long)colour * 8 * hn;
-    const long long sy = L.X, sz = (long long)L.X * L.Y;
-    const double s = a[h] * p[q - 1] + a[hn + h] * p[q + 1] + a[2 * hn + h] * p[q - sy] +
-                     a[3 * hn + h] * p[q + sy] + a[4 * hn + h] * p[q - sz] +
-                     a[5 * hn + h] * p[q + sz] + a[7 * hn + h];
-    p[q] = (1.0 - beta) * p[q] + beta / a[6 * hn + h] * s;
-}
-
 // 256-thread block sum / max (t: linear thread id, wavefronts of 64
 // consecutive ids), result in thread 0 (sm: 4 doubles)
 __device__ __forceinline__ double blk_red(double v, double *sm, bool mx, int t) {
@@ -126,22 +105,31 @@ __device__ __forceinline__ double blk_red(double v, double *sm, bool mx, int t) 
     return r;
 }
 
-// FreeSolver on the colour-split A, the residual statistics fused into the
-// sweep: the cells of one colour (64 x 4 pair tiles, the planes strided by
-// gridDim.z), with
-// UPDATE the RB-SOR update of k_rb_pass_split first.  Every neighbour of a
-// cell has the other colour, so after the second pass both the cells it
-// updated (UPDATE) and, in a pass of its own, the first colour's cells see
-// final values: their statistics equal k_resid_stats_fs's (same residual
-// expression, sums in another order).  Block partials {sum r^2, max |r|,
-// active cells, NaN cells} at part[c * kRedBlocks + boff + block].
-// !FS (NewSolver_std): every cell, the residual of MGsolver.f90:97-100 as
-// compute_residual_norm forms it, partial 0 = sum |r|^norm.
-template <bool UPDATE, bool FS = true>
+// FreeSolver (FS) and NewSolver_std (!FS) on the colour-split A, the residual
+// statistics fused into the sweep: the cells of one colour (64 x 4 pair
+// tiles, the planes strided by gridDim.z).  Every neighbour of a cell has the
+// other colour, so after an iteration's second pass both the cells it
+// updated (PASS_SECOND: the RB-SOR update of k_rb_pass, then the residual)
+// and the first colour's cells see final values.  The latter's residuals are
+// formed by the next iteration's first pass, before its update, from the
+// values that the update reads anyway (PASS_FIRST; it keeps what it
+// overwrites in old, one value a pair, for an iteration that turns out to be
+// the last one); after the last iteration, in a pass of their own
+// (PASS_STATS).  128^3: 53 us an iteration's passes against 73 with a
+// statistics pass of its own in every one (67 MB of A each).
+// The statistics equal k_resid_stats_fs's (same residual expression, sums
+// in another order).  Block partials {sum r^2, max |r|, active cells, NaN
+// cells} at part[c * kRedBlocks + boff + block].  !FS: every cell, the
+// residual of MGsolver.f90:97-100 as compute_residual_norm forms it, partial
+// 0 = sum |r|^norm.  Nothing is done once *stop is set.
+enum { PASS_FIRST, PASS_SECOND, PASS_STATS };
+template <int PASS, bool FS>
 __global__ void __launch_bounds__(256)
-k_fs_pass_stats(LvlK L, const double *__restrict__ As, double *__restrict__ p,
+k_sor_pass(LvlK L, const double *__restrict__ As, double *__restrict__ p,
                 const int *__restrict__ pcmask, int flag, double beta, int colour,
-                double *__restrict__ part, int boff, int norm = 2) {
+                double *__restrict__ part, int boff, int norm, double *__restrict__ old,
+                const int *__restrict__ stop) {
+    if (*stop) return;
     __shared__ double sm[4];
     const long long hn = lk_cells(L) / 2;
     const int hx = L.nx / 2;
@@ -158,24 +146,26 @@ k_fs_pass_stats(LvlK L, const double *__restrict__ As, double *__restrict__ p,
             if (!(flag == 1 ? mk == 0 : (mk == 1 || mk == 2))) continue;
         }
         double pc = p[q];
-        if (UPDATE) {
-            const double s = a[h] * p[q - 1] + a[hn + h] * p[q + 1] + a[2 * hn + h] * p[q - sy] +
-                             a[3 * hn + h] * p[q + sy] + a[4 * hn + h] * p[q - sz] +
-                             a[5 * hn + h] * p[q + sz] + a[7 * hn + h];
-            pc = (1.0 - beta) * pc + beta / a[6 * hn + h] * s;
-            p[q] = pc;
+        const double pw = p[q - 1], pe = p[q + 1], ps = p[q - sy], pn = p[q + sy], pb = p[q - sz],
+                     pt = p[q + sz];
+        double pnew = pc;
+        if (PASS != PASS_STATS) {
+            const double s = a[h] * pw + a[hn + h] * pe + a[2 * hn + h] * ps + a[3 * hn + h] * pn +
+                             a[4 * hn + h] * pb + a[5 * hn + h] * pt + a[7 * hn + h];
+            pnew = (1.0 - beta) * pc + beta / a[6 * hn + h] * s;
+            p[q] = pnew;
         }
+        if (PASS == PASS_FIRST) old[h] = pc;
+        if (PASS == PASS_SECOND) pc = pnew;
         if (!FS) {
-            const double r = fabs(a[7 * hn + h] - a[6 * hn + h] * pc + a[h] * p[q - 1] +
-                                  a[hn + h] * p[q + 1] + a[2 * hn + h] * p[q - sy] +
-                                  a[3 * hn + h] * p[q + sy] + a[4 * hn + h] * p[q - sz] +
-                                  a[5 * hn + h] * p[q + sz]);
+            const double r = fabs(a[7 * hn + h] - a[6 * hn + h] * pc + a[h] * pw + a[hn + h] * pe +
+                                  a[2 * hn + h] * ps + a[3 * hn + h] * pn + a[4 * hn + h] * pb +
+                                  a[5 * hn + h] * pt);
             s2 += norm == 1 ? r : (norm == 2 ? r * r : pow(r, (double)norm));
             continue;
         }
-        const double r = fabs(-pc * a[6 * hn + h] + a[h] * p[q - 1] + a[hn + h] * p[q + 1] +
-                              a[2 * hn + h] * p[q - sy] + a[3 * hn + h] * p[q + sy] +
-                              a[4 * hn + h] * p[q - sz] + a[5 * hn + h] * p[q + sz] + a[7 * hn + h]);
+        const double r = fabs(-pc * a[6 * hn + h] + a[h] * pw + a[hn + h] * pe + a[2 * hn + h] * ps +
+                              a[3 * hn + h] * pn + a[4 * hn + h] * pb + a[5 * hn + h] * pt + a[7 * hn + h]);
         bool nan = r != r;
 #pragma unroll
         for (int s = 0; s < 8; ++s) nan |= a[s * hn + h] != a[s * hn + h];
@@ -188,12 +178,76 @@ k_fs_pass_stats(LvlK L, const double *__restrict__ As, double *__restrict__ p,
     const long long b = boff + blockIdx.x + (long long)gridDim.x * (blockIdx.y + (long long)gridDim.y * blockIdx.z);
     double v = blk_red(s2, sm, false, t);
     if (t == 0) part[b] = v;
+    if (!FS) return;
     v = blk_red(mx, sm, true, t);
     if (t == 0) part[kRedBlocks + b] = v;
     v = blk_red(cnt, sm, false, t);
     if (t == 0) part[2 * kRedBlocks + b] = v;
     v = blk_red(bad, sm, false, t);
     if (t == 0) part[3 * kRedBlocks + b] = v;
+}
+
+// An iteration's totals from the block partials, one wavefront group of 256
+// threads a component (FS: sum r^2, max |r|, active cells, NaN cells; !FS:
+// sum |r|^norm), into the host's slot (seq last, with a system-scope
+// release), and the reference's decision: diverged or converged sets *stop
+// for the passes already queued behind.  (One component after another in
+// 256 threads took 18.7 us for 4096 partials.)
+template <bool FS>
+__global__ void __launch_bounds__(1024)
+k_sor_final(const double *__restrict__ part, int nblocks, double N, int norm, double maxError,
+            SorBox *box, unsigned long long seq, int *stop) {
+    if (*stop) return;
+    __shared__ double sm[16], out[4];
+    const int c = threadIdx.x >> 8, t = threadIdx.x & 255;
+    const bool mx = c == 1;
+    double v = mx ? -INFINITY : 0.0;
+    if (FS || c == 0)
+        for (int b0 = t; b0 < nblocks; b0 += 16 * 256) {
+            double x[16];   // all loads before the first use
+#pragma unroll
+            for (int q = 0; q < 16; ++q)
+                x[q] = b0 + q * 256 < nblocks ? part[c * kRedBlocks + b0 + q * 256] : (mx ? -INFINITY : 0.0);
+#pragma unroll
+            for (int q = 0; q < 16; ++q) v = mx ? fmax(v, x[q]) : v + x[q];
+        }
+    const double r = blk_red(v, sm + 4 * c, mx, t);
+    if (t == 0) out[c] = r;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        bool bad, done;
+        if (FS) {   // catch_divergence_fs with one rank; use_L_inf
+            bad = out[3] > 0.0 || !(out[0] <= 1e18);
+            done = out[1] < maxError;
+        } else {
+            const double res2 = out[0] / N;
+            bad = !(res2 <= 1e16);   // > 1e16 or NaN
+            done = (norm == 2 ? sqrt(res2) : res2) < maxError;
+        }
+        for (int q = 0; q < 4; ++q) box->st[q] = out[q];
+        box->bad = bad ? 1.0 : 0.0;
+        box->stop = bad || done ? 1.0 : 0.0;
+        if (bad || done) *stop = 1;
+        __hip_atomic_store(&box->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
+// the first colour's values before the last PASS_FIRST
+template <bool FS>
+__global__ void __launch_bounds__(256)
+k_sor_undo(LvlK L, double *__restrict__ p, const int *__restrict__ pcmask, int flag,
+           const double *__restrict__ old) {
+    const int j = blockIdx.y * blockDim.y + threadIdx.y;
+    const int k = blockIdx.z;
+    const int m = blockIdx.x * blockDim.x + threadIdx.x;
+    if (j >= L.ny || m >= L.nx / 2) return;
+    const long long q = ipad(L, 2 * m + ((j + k) & 1), j, k);
+    if (FS && !(flag == 1 ? pcmask[q] == 0 : (pcmask[q] == 1 || pcmask[q] == 2))) return;
+    p[q] = old[((long long)k * L.ny + j) * (L.nx / 2) + m];
+}
+
+__global__ void __launch_bounds__(64) k_sor_start(int *stop) {
+    if (threadIdx.x == 0) *stop = 0;
 }
 
 // One-layer periodic wrap of the face ghosts of a level.
@@ -494,6 +548,97 @@ int ref_solve(pps_handle *h, const double *dA, double *dp, double maxError,
     return PPS_OK;
 }
 
+// RB-SOR iterations on the colour-split A for at most maxit iterations: on
+// the stream, iteration k's first pass (which also forms the statistics of
+// iteration k-1's first colour), the totals of iteration k-1, iteration k's
+// second pass.  The host queues kSorAhead iterations beyond the one whose
+// totals it waits for, so the device does not idle while they travel: once
+// the totals set the stop flag the passes behind them return at once, and
+// the one first pass that ran before them is undone.  Gives the iteration
+// that stopped (0: none did) and the totals of the last one; each
+// iteration's totals are passed to `seen`.
+constexpr int kSorAhead = 2;
+static_assert(kSorAhead + 2 <= kSorBoxes, "a slot for every iteration in flight");
+template <bool FS, class Seen>
+static int sor_split(pps_handle *h, const LvlK &L, const double *As, double *dp, const int *dmask, int flag,
+                     double beta, int maxit, double N, int norm, double maxError, int nbk, const dim3 &tgrid,
+                     const dim3 &sgrid, hipStream_t s, int *stopped, bool *bad, Seen seen) {
+    double *part = stats_partials(h);
+    if (!part) return PPS_ERR_HIP;
+    int *stop = stats_flag(h);
+    const long long hn = (long long)L.nx * L.ny * L.nz / 2;
+    PPS_TRY(h->sorold.ensure(sizeof(double) * (size_t)hn));
+    double *old = h->sorold.as<double>();
+    if (!h->sorbox) {
+        PPS_HIP(hipHostMalloc((void **)&h->sorbox, kSorBoxes * sizeof(SorBox), hipHostMallocCoherent));
+        for (int q = 0; q < kSorBoxes; ++q) h->sorbox[q].seq = 0;
+    }
+    k_sor_start<<<1, 64, 0, s>>>(stop);
+    const unsigned long long base = h->sorseq;
+    h->sorseq += (unsigned long long)maxit;
+    auto box = [&](int k) { return h->sorbox + (base + k) % kSorBoxes; };
+    auto totals = [&](int k) {
+        k_sor_final<FS><<<1, 1024, 0, s>>>(part, 2 * nbk, N, norm, maxError, box(k), base + k, stop);
+    };
+    auto queue = [&](int k) {
+        k_sor_pass<PASS_FIRST, FS><<<tgrid, kCellBlock, 0, s>>>(L, As, dp, dmask, flag, beta, 0, part, nbk, norm,
+                                                               old, stop);
+        launch_halo(L, dp, s);
+        if (k > 1) totals(k - 1);
+        k_sor_pass<PASS_SECOND, FS><<<tgrid, kCellBlock, 0, s>>>(L, As, dp, dmask, flag, beta, 1, part, 0, norm,
+                                                                old, stop);
+        launch_halo(L, dp, s);
+        if (k == maxit) {
+            k_sor_pass<PASS_STATS, FS><<<tgrid, kCellBlock, 0, s>>>(L, As, dp, dmask, flag, beta, 0, part, nbk,
+                                                                   norm, old, stop);
+            totals(k);
+        }
+    };
+    *stopped = 0;
+    *bad = false;
+    int queued = 0;
+    for (int k = 1; k <= maxit; ++k) {
+        // iteration k's totals come with iteration k+1's first pass
+        while (queued < maxit && queued < k + kSorAhead) queue(++queued);
+        PPS_HIP(hipGetLastError());
+        const SorBox *b = box(k);
+        for (long long spin = 1; __atomic_load_n(&b->seq, __ATOMIC_ACQUIRE) != base + k; ++spin) {
+            if ((spin & 255) == 0) {
+                const hipError_t e = hipStreamQuery(s);
+                if (e == hipSuccess && __atomic_load_n(&b->seq, __ATOMIC_ACQUIRE) != base + k) {
+                    std::fprintf(stderr, "libpps: the stream drained without the expected reduction\n");
+                    return PPS_ERR_HIP;
+                }
+                if (e != hipSuccess && e != hipErrorNotReady) PPS_HIP(e);
+            }
+            __builtin_ia32_pause();
+        }
+        seen(b->st);
+        if (b->stop != 0.0) {
+            *stopped = k;
+            *bad = b->bad != 0.0;
+            if (k < maxit) {
+                k_sor_undo<FS><<<sgrid, kCellBlock, 0, s>>>(L, dp, dmask, flag, old);
+                launch_halo(L, dp, s);
+                PPS_HIP(hipGetLastError());
+            }
+            break;
+        }
+    }
+    return PPS_OK;
+}
+
+// Launch shapes of the split passes: the planes strided so that a pass has at
+// most about 2048 blocks, one partial slot each.  False: too many row tiles
+// (the interleaved path runs).
+static bool sor_shapes(const LvlK &L, dim3 *sgrid, dim3 *tgrid, int *nbk) {
+    *sgrid = dim3((unsigned)((L.nx / 2 + 63) / 64), (unsigned)((L.ny + 3) / 4), (unsigned)L.nz);
+    const long long tiles = (long long)sgrid->x * sgrid->y;
+    *tgrid = dim3(sgrid->x, sgrid->y, (unsigned)std::max<long long>(1, std::min<long long>(L.nz, 2048 / tiles)));
+    *nbk = (int)(tiles * tgrid->z);
+    return 2LL * *nbk <= kRedBlocks;
+}
+
 // NewSolver_std (newsolver.f90:78-174) with catch_divergence folded into
 // the residual norm: NaN in A or p makes the norm NaN.
 int sor_solve(pps_handle *h, const double *dA, double *dp, double maxError,
@@ -508,33 +653,27 @@ int sor_solve(pps_handle *h, const double *dA, double *dp, double maxError,
     int rc = PPS_OK;
     const double *As = split_colours(h, L, dA, s, &rc);
     PPS_TRY(rc);
-    // split path: pass 0, halo, pass 1 + its cells' residuals, halo, the
-    // residuals of pass 0's cells (the planes strided: ~2048 blocks each)
-    const dim3 sgrid((unsigned)((L.nx / 2 + 63) / 64), (unsigned)((L.ny + 3) / 4), (unsigned)L.nz);
-    const long long tiles = (long long)sgrid.x * sgrid.y;
-    const dim3 tgrid(sgrid.x, sgrid.y, (unsigned)std::max<long long>(1, std::min<long long>(L.nz, 2048 / tiles)));
-    const int nbk = (int)(tiles * tgrid.z);
-    if (As && 2LL * nbk > kRedBlocks) As = nullptr;
-    double *part = As ? stats_partials(h) : nullptr;
-    if (As && !part) return PPS_ERR_HIP;
-    int k;
+    dim3 sgrid, tgrid;
+    int nbk = 0, k;
+    if (As && sor_shapes(L, &sgrid, &tgrid, &nbk)) {
+        double res2 = 0.0;
+        int stopped;
+        bool bad;
+        PPS_TRY(sor_split<false>(h, L, As, dp, nullptr, 0, beta, maxit, N, norm, maxError, nbk, tgrid, sgrid, s,
+                                 &stopped, &bad, [&](const double *st) {
+                                     res2 = st[0] / N;
+                                     t2 = norm == 2 ? std::sqrt(res2) : res2;
+                                     if (res2 <= 1e16) h->hist.push_back(t2);
+                                 }));
+        *it = stopped ? stopped : maxit + 1;
+        *tres2 = bad ? res2 : t2;
+        return bad ? PPS_ERR_DIVERGED : PPS_OK;
+    }
     for (k = 1; k <= maxit; ++k) {
-        if (As) {
-            k_rb_pass_split<<<sgrid, kCellBlock, 0, s>>>(L, As, dp, nullptr, 0, beta, 0);
-            launch_halo(L, dp, s);
-            k_fs_pass_stats<true, false><<<tgrid, kCellBlock, 0, s>>>(L, As, dp, nullptr, 0, beta, 1, part, 0,
-                                                                      norm);
-            launch_halo(L, dp, s);
-            k_fs_pass_stats<false, false><<<tgrid, kCellBlock, 0, s>>>(L, As, dp, nullptr, 0, beta, 0, part,
-                                                                       nbk, norm);
-            PPS_HIP(hipGetLastError());
-            PPS_TRY(stats_finish(h, 2 * nbk, 1, 0, &res, s));
-        } else {
-            launch_relax(L, dA, dp, beta, s);
-            launch_halo(L, dp, s);
-            PPS_HIP(hipGetLastError());
-            PPS_TRY(compute_residual_norm(h, D, dA, dp, norm, &res, s));
-        }
+        launch_relax(L, dA, dp, beta, s);
+        launch_halo(L, dp, s);
+        PPS_HIP(hipGetLastError());
+        PPS_TRY(compute_residual_norm(h, D, dA, dp, norm, &res, s));
         double res2 = res / N;
         if (!(res2 <= 1e16)) {  // > 1e16 or NaN
             *it = k;
@@ -615,37 +754,31 @@ int free_solve(pps_handle *h, const double *dA, double *dp, const int *dmask, co
     int rc = PPS_OK;
     const double *As = split_colours(h, L, dA, s, &rc);
     PPS_TRY(rc);
-    int k;
-    // split path: pass 0, halo, pass 1 + its cells' statistics, halo, the
-    // statistics of pass 0's cells
-    // (the statistics kernels stride the planes so that each has at most
-    // ~2048 blocks, one partial slot each)
-    const dim3 sgrid((unsigned)((L.nx / 2 + 63) / 64), (unsigned)((L.ny + 3) / 4), (unsigned)L.nz);
-    const long long tiles = (long long)sgrid.x * sgrid.y;
-    const dim3 tgrid(sgrid.x, sgrid.y, (unsigned)std::max<long long>(1, std::min<long long>(L.nz, 2048 / tiles)));
-    const int nbk = (int)(tiles * tgrid.z);
-    if (As && 2LL * nbk > kRedBlocks) As = nullptr;   // too many row tiles: interleaved path
-    double *part = As ? stats_partials(h) : nullptr;
-    if (As && !part) return PPS_ERR_HIP;
+    dim3 sgrid, tgrid;
+    int nbk = 0, k;
+    if (As && sor_shapes(L, &sgrid, &tgrid, &nbk)) {
+        double sum = 0.0;
+        int stopped;
+        bool bad;
+        PPS_TRY(sor_split<true>(h, L, As, dp, dmask, solver_flag, beta, maxit, 1.0, 2, maxError, nbk, tgrid, sgrid,
+                                s, &stopped, &bad, [&](const double *st) {
+                                    sum = st[0];
+                                    if (st[3] > 0.0 || !(st[0] <= 1e18)) return;
+                                    t2 = std::sqrt(st[0]) / st[2];
+                                    h->hist.push_back(t2);
+                                }));
+        *it = stopped ? stopped : maxit + 1;
+        *tres2 = bad ? sum : t2;
+        return bad ? PPS_ERR_DIVERGED : PPS_OK;
+    }
     for (k = 1; k <= maxit; ++k) {
         double st[4];
-        if (As) {
-            k_rb_pass_split<<<sgrid, kCellBlock, 0, s>>>(L, As, dp, dmask, solver_flag, beta, 0);
-            launch_halo(L, dp, s);
-            k_fs_pass_stats<true><<<tgrid, kCellBlock, 0, s>>>(L, As, dp, dmask, solver_flag, beta, 1, part, 0);
-            launch_halo(L, dp, s);
-            k_fs_pass_stats<false><<<tgrid, kCellBlock, 0, s>>>(L, As, dp, dmask, solver_flag, beta, 0, part,
-                                                                nbk);
-            PPS_HIP(hipGetLastError());
-            PPS_TRY(stats_finish(h, 2 * nbk, 4, 1 << 1, st, s));
-        } else {
-            k_rb_pass_fs<<<grid, kCellBlock, 0, s>>>(L, dA, dp, dmask, solver_flag, beta, 0);
-            launch_halo(L, dp, s);
-            k_rb_pass_fs<<<grid, kCellBlock, 0, s>>>(L, dA, dp, dmask, solver_flag, beta, 1);
-            launch_halo(L, dp, s);
-            PPS_HIP(hipGetLastError());
-            PPS_TRY(fs_residual_stats(h, D, dA, dp, dmask, solver_flag, st, s));
-        }
+        k_rb_pass_fs<<<grid, kCellBlock, 0, s>>>(L, dA, dp, dmask, solver_flag, beta, 0);
+        launch_halo(L, dp, s);
+        k_rb_pass_fs<<<grid, kCellBlock, 0, s>>>(L, dA, dp, dmask, solver_flag, beta, 1);
+        launch_halo(L, dp, s);
+        PPS_HIP(hipGetLastError());
+        PPS_TRY(fs_residual_stats(h, D, dA, dp, dmask, solver_flag, st, s));
         if (st[3] > 0.0 || !(st[0] <= 1e18)) {
             *it = k;
             *tres2 = st[0];

@@ -88,3 +88,40 @@ def test_free_solver_host_entry_point_and_errors(pps, orc):
         og.interior(m2)[3, 4, 5] = 0
         with pytest.raises(pps.PPSError):
             s.free_solver(B, p0.copy(), m2, pgas, 1, tol)
+
+
+@pytest.mark.parametrize("shape,bc", [((64, 40, 24), (0,) * 6), ((130, 9, 33), (0,) * 6),
+                                      ((32, 36, 70), (1, 0, 0, 1, 0, 0))])
+@pytest.mark.parametrize("maxit", [1, 2, 7])
+def test_free_solver_stops_where_the_oracle_does(pps, orc, shape, bc, maxit):
+    """Iterations run ahead of their stopping test on the device: p must be
+    that of the iteration it stops at, whether the limit ends it (maxit) or the
+    residual does (a tolerance met one iteration before the limit)."""
+    _say("free solver stop", shape, bc, maxit)
+    g = pps.Grid.make(*shape, bdry_cond=bc)
+    og = orc.OrcGrid.make(*shape, bc=bc)
+    rho, u, v, w = pps.synth_fields(g, [(0.4, 0.5, 0.6, 0.25)], 1.0, 100.0, 1.5, seed=3)
+    um, vm, wm = pps.pressure_masks(g)
+    At = pps.setup_poisson(g, u, v, w, um, vm, wm, rho, 1.0)
+    pps.remove_rhs_mean(g, At)
+    A = _host(At)
+    rng = np.random.default_rng(3)
+    m = np.zeros(og.shape_p, dtype=np.int32)
+    og.interior(m)[...] = (rng.random(og.interior(m).shape) < 0.2).astype(np.int32)
+    pgas = np.zeros(og.shape_p)
+    pr = np.zeros(og.shape_p)
+    rc, it, t2, hist = orc.free_solver(og, A, pr, m, pgas, 1, 0.0, 1.2, maxit)
+    # the max-norm residual of that last iterate: a tolerance just above it is
+    # met by this iteration and (the residual falls) by none before
+    act = (og.interior(m) == 0)
+    res = np.abs(np.where(act, orc.residual_field(og, A, pr), 0.0)).max()
+    for tol, limit in ((0.0, maxit), (res * 1.0000001, maxit + 3)):
+        with pps.Solver(g, method="sor") as s:
+            p = torch.zeros(g.shape_p, dtype=torch.float64, device="cuda")
+            git, gt2 = s.free_solve(At, p, torch.from_numpy(m).cuda(), torch.from_numpy(pgas).cuda(), 1, tol,
+                                    1.2, limit)
+            n_hist = len(s.history())
+        assert git == (maxit + 1 if tol == 0.0 else maxit)
+        assert n_hist == maxit
+        assert np.array_equal(og.interior(_host(p)), og.interior(pr))
+        assert gt2 == pytest.approx(t2, rel=1e-12)
