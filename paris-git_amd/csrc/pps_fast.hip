@@ -38,6 +38,7 @@
 #include "pps_level.h"
 #include "pps_march.h"
 #include "pps_row.h"
+#include "pps_scal.h"
 #include "pps_tail.h"
 #include "pps_xcd.h"
 
@@ -1415,15 +1416,8 @@ k_tail_tri(TailTriK<T> K) {
 }
 
 // ---------------------------------------------------------------------
-// FP64 outer iteration kernels.  Scalars live on the device:
+// FP64 outer iteration kernels
 // ---------------------------------------------------------------------
-enum { S_RZ = 0, S_ZMEAN, S_BETA, S_DQ, S_ALPHA, S_RR, S_BB, S_FIRST, S_STOP, S_N };
-// alpha of the direction in ring slot j: S[S_AH + j] (j < kRingSlots;
-// the scalars take 64 doubles)
-constexpr int kRingSlots = 9;   // directions held for deferred x updates
-constexpr int S_AH = S_N;
-static_assert(S_AH + kRingSlots <= 64, "ring alphas fit the scalars");
-
 // 2.5-D launch shape for z-marching kernels: (64, 4) threads over (x, y),
 // each thread walks `zc` consecutive planes; at most kRedBlocks blocks so
 // that one partial slot per block suffices.
@@ -1446,25 +1440,6 @@ static ZGrid zgrid(int nx, int ny, int nz, int target = 16384) {
     z.blocks = (int)(cols * chunks);
     return z;
 }
-// fixed-order sum of nb partials, the same value in every thread (any
-// block of at most 1024 threads whose x extent is a multiple of 64)
-__device__ __forceinline__ double sum_partials(const double *part, int nb) {
-    __shared__ double sm[16];
-    const int nt = blockDim.x * blockDim.y * blockDim.z;
-    const int tid = threadIdx.x + blockDim.x * (threadIdx.y + blockDim.y * threadIdx.z);
-    const int nw = nt >> 6;
-    double v = 0.0;
-    for (int b = tid; b < nb; b += nt) v += part[b];
-    v = wsum(v);
-    if ((tid & 63) == 0) sm[tid >> 6] = v;
-    __syncthreads();
-    double t = 0.0;
-    for (int w = 0; w < nw; ++w) t += sm[w];
-    __syncthreads();
-    return t;
-}
-
-
 // FP64 fine operator for the outer iteration: +x/+y/+z couplings and the
 // diagonal, either the compact planes the setup pass writes (0 on wall
 // faces) or the caller's A slots 2, 4, 6, 7 (mixed mode), whose wall-face
@@ -1572,11 +1547,13 @@ k_dot_rz(long long n, const double *__restrict__ r, const TZ *__restrict__ z, do
 // buffers: the plane written at step s+1 was last read at step s-2).
 // Registers held to 64 a thread (two blocks a CU): the FP64 form needs 66
 // otherwise, one block a CU, and ran 239 against 223 us at 256^3.
-template <class TZ, bool DGI>
+// FOLD: beta from its partials here (bk.nb of them), else from S (the sums
+// cost registers, which this form has none to spare of).
+template <class TZ, bool DGI, bool FOLD>
 __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8)))
 k_dq_tiled(OpK L, TGrid g, const TZ *__restrict__ z, const TZ *__restrict__ dold,
            TZ *__restrict__ dnew, double *__restrict__ q, double *__restrict__ x,
-           const double *__restrict__ S, double *__restrict__ part) {
+           double *__restrict__ S, double *__restrict__ part, BetaK bk) {
     __shared__ double D[3][18][66];
     const int nx = L.nx, ny = L.ny, nz = L.nz;
     const int bid = xcd_order(blockIdx.x, gridDim.x);
@@ -1585,7 +1562,19 @@ k_dq_tiled(OpK L, TGrid g, const TZ *__restrict__ z, const TZ *__restrict__ dold
     const int i = tx * 64 + li, j = ty * 16 + lj;
     const int k0 = ch * g.zc, k1 = min(k0 + g.zc, nz);
     const bool in = i < nx && j < ny;
-    const double beta = S[S_BETA], zm = S[S_ZMEAN], ax = S[S_ALPHA];
+    double beta, zm;
+    if constexpr (FOLD) {
+        double sums[3], rho;
+        sum_partials3(part, bk.nb, sums);
+        beta_of(bk, sums, S, &beta, &zm, &rho);
+        beta = uniform(beta);
+        zm = uniform(zm);
+        if (blockIdx.x == 0 && threadIdx.x + threadIdx.y == 0) S[bk.wr] = rho;
+    } else {
+        beta = S[S_BETA];
+        zm = S[S_ZMEAN];
+    }
+    const double ax = S[S_ALPHA];
     // x null: the previous direction is not applied here (the caller
     // defers it)
     const bool use_old = beta != 0.0, upd = x && ax != 0.0;
@@ -1679,7 +1668,8 @@ k_dq_tiled(OpK L, TGrid g, const TZ *__restrict__ z, const TZ *__restrict__ dold
         zo1 = zo2; do1 = do2; zh1 = zh2; dh1 = dh2;
         __syncthreads();
     }
-    block_partial(dq, part);
+    // slot 3: other blocks may still read slots 0 to 2
+    block_partial(dq, part + 3 * kRedBlocks);
 }
 
 
@@ -1688,8 +1678,19 @@ k_dq_tiled(OpK L, TGrid g, const TZ *__restrict__ z, const TZ *__restrict__ dold
 template <class TB>
 __global__ void __launch_bounds__(256)
 k_update(long long n, double *__restrict__ r, const double *__restrict__ q, TB *__restrict__ bt,
-         const double *__restrict__ S, double *__restrict__ part) {
-    const double alpha = S[S_ALPHA];
+         double *__restrict__ S, double *__restrict__ part, AlphaK ak) {
+    double alpha;
+    if (ak.nb) {   // uniform
+        const double dq = sum_partials(part + 3 * kRedBlocks, ak.nb);
+        alpha = uniform(S[ak.rz] / dq);
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            S[S_DQ] = dq;
+            S[S_ALPHA] = alpha;
+            S[S_AH + ak.slot] = alpha;
+        }
+    } else {
+        alpha = S[S_ALPHA];
+    }
     double rr = 0.0;
     for (long long c = blockIdx.x * 256LL + threadIdx.x; c < n; c += (long long)gridDim.x * 256) {
         // r and q non-temporal; the FP32 copy of r, which the next V-cycle's
@@ -1730,16 +1731,6 @@ k_resid_zero(long long n, const double *__restrict__ b, double *__restrict__ r, 
     block_partial(rr, part + kRedBlocks);
 }
 
-// the outer iteration's scalars at its start: first iteration, no pending
-// x update, not stopped
-__global__ void __launch_bounds__(64) k_outer_start(double *__restrict__ S) {
-    if (threadIdx.x == 0) {
-        S[S_FIRST] = 1.0;
-        S[S_ALPHA] = 0.0;
-        S[S_STOP] = 0.0;
-    }
-}
-
 // refinement step: x += z - zmean ; partial sums of z
 template <class TZ>
 __global__ void __launch_bounds__(256)
@@ -1761,33 +1752,29 @@ k_add_z(long long n, double *__restrict__ x, const TZ *__restrict__ z, const dou
         x[c] += (double)z[c] - zm;
 }
 
-// the beta step from k_dot_rz's partials: zmean, rho = r.(z - zmean),
-// beta = rho / rho_old
+// the beta step
 __global__ void __launch_bounds__(1024)
-k_scal_beta(const double *__restrict__ part, int nb, long long n, int singular,
-            double *__restrict__ S) {
-    const double rz = sum_partials(part, nb);
-    const double zs = sum_partials(part + kRedBlocks, nb);
-    const double rs = sum_partials(part + 2 * kRedBlocks, nb);
+k_scal_beta(const double *__restrict__ part, BetaK bk, double *__restrict__ S) {
+    double sums[3];
+    sum_partials3(part, bk.nb, sums);
     if (threadIdx.x == 0) {
-        const double zm = singular ? zs / (double)n : 0.0;
-        const double rho = rz - zm * rs;
-        const double first = S[S_FIRST];
-        S[S_BETA] = first != 0.0 ? 0.0 : rho / S[S_RZ];
-        S[S_RZ] = rho;
+        double beta, zm, rho;
+        beta_of(bk, sums, S, &beta, &zm, &rho);
+        S[S_BETA] = beta;
+        S[bk.wr] = rho;
         S[S_ZMEAN] = zm;
-        S[S_FIRST] = 0.0;
     }
 }
 
-// the alpha step from k_dq's partials
+// the alpha step from k_dq_tiled's partials
 __global__ void __launch_bounds__(1024)
-k_scal_alpha(const double *__restrict__ part, int nb, double *__restrict__ S, int slot) {
-    const double dq = sum_partials(part, nb);
+k_scal_alpha(const double *__restrict__ part, AlphaK ak, double *__restrict__ S) {
+    const double dq = sum_partials(part + 3 * kRedBlocks, ak.nb);
     if (threadIdx.x == 0) {
+        const double alpha = S[ak.rz] / dq;
         S[S_DQ] = dq;
-        S[S_ALPHA] = S[S_RZ] / dq;
-        S[S_AH + slot] = S[S_ALPHA];
+        S[S_ALPHA] = alpha;
+        S[S_AH + ak.slot] = alpha;
     }
 }
 
@@ -1837,8 +1824,12 @@ k_sub_mean(long long n, double *__restrict__ b, const double *__restrict__ part,
     for (long long c = blockIdx.x * 256LL + threadIdx.x; c < n; c += (long long)gridDim.x * 256) b[c] -= m;
 }
 
+// r.r (and b.b): the sums, and given a mailbox the host's copy of them with
+// the setup flags and the stopping test (tol > 0), which a first sweep already
+// queued behind this kernel reads from S.  start: an outer iteration starts
+// from here (no pending x update, not stopped).
 __global__ void __launch_bounds__(1024)
-k_scal_rr(const double *__restrict__ part, int nb, int with_bb, double *__restrict__ S,
+k_scal_rr(const double *__restrict__ part, int nb, int with_bb, double *__restrict__ S, int start,
           Mailbox *mb = nullptr, unsigned long long seq = 0, const int *flags = nullptr,
           double N = 1.0, double tol = 0.0) {
     const double rr = sum_partials(part, nb);
@@ -1847,20 +1838,13 @@ k_scal_rr(const double *__restrict__ part, int nb, int with_bb, double *__restri
     if (threadIdx.x == 0) {
         S[S_RR] = rr;
         if (with_bb) S[S_BB] = bb;
-        // the outer iteration's stopping test, sqrt(rr / N) < tol (tol > 0),
-        // for the first sweep already queued behind this kernel; the host
-        // takes the same decision from the mailbox
         const double stop = (tol > 0.0 && sqrt(rr / N) < tol) ? 1.0 : 0.0;
         if (tol > 0.0) S[S_STOP] = stop;
-        if (mb) {
-            // the values, then seq with a system-scope release: a host that
-            // reads seq (acquire) sees them
-            mb->rr = rr;
-            mb->bb = bb;
-            mb->flags = flags ? (double)*flags : 0.0;
-            mb->pad = stop;
-            __hip_atomic_store(&mb->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+        if (start) {
+            S[S_ALPHA] = 0.0;
+            S[S_STOP] = 0.0;
         }
+        if (mb) post(mb, seq, rr, bb, flags ? (double)*flags : 0.0, stop);
     }
 }
 
@@ -2827,13 +2811,13 @@ static LegK leg_grid(const Level<T> &L, int ez, const Cycle &cy) {
 }
 template <class T>
 static void leg_pre(const Level<T> &L, const Level<T> &C, const T *b, const Cycle &cy, hipStream_t s,
-                    const double *skip = nullptr) {
+                    const StopK &stop = StopK{}) {
     const int ez = leg_ez(L, cy);
     const LegK g = leg_grid(L, ez, cy);
     auto k = cy.dgi ? k_leg_pre<T, true, 16> : k_leg_pre<T, false, 16>;
     if constexpr (sizeof(T) == 4)
         if (ez == 24) k = cy.dgi ? k_leg_pre<T, true, 24> : k_leg_pre<T, false, 24>;
-    k<<<g.tx * g.ty * g.tz, kLegThreads, 0, s>>>(L.k(), g, L.g, b, L.x, C.b, skip);
+    k<<<g.tx * g.ty * g.tz, kLegThreads, 0, s>>>(L.k(), g, L.g, b, L.x, C.b, stop);
 }
 // dot: block partials, as rb_sweep's (returns their block count)
 template <class T>
@@ -2889,11 +2873,11 @@ static MarchK march_grid(const Level<T> &L, const Cycle &cy, int *blocks) {
 }
 template <class T>
 static void march_pre(const Level<T> &L, const Level<T> &C, const T *b, const Cycle &cy, hipStream_t s,
-                      const double *skip = nullptr) {
+                      const StopK &stop = StopK{}) {
     int blocks;
     const MarchK g = march_grid(L, cy, &blocks);
     auto k = L.nx % (16 / (int)sizeof(T)) == 0 ? k_march<T, true, false, true> : k_march<T, true, false, false>;
-    k<<<blocks, kMarchThreads, 0, s>>>(L.k(), g, L.g, b, nullptr, nullptr, L.x, C.b, nullptr, skip);
+    k<<<blocks, kMarchThreads, 0, s>>>(L.k(), g, L.g, b, nullptr, nullptr, L.x, C.b, nullptr, stop);
 }
 template <class T>
 static int march_post(Level<T> &L, int l, const Level<T> &C, const T *b, const Cycle &cy, Prof *prof, hipStream_t s,
@@ -2909,21 +2893,27 @@ static int march_post(Level<T> &L, int l, const Level<T> &C, const T *b, const C
     hipEvent_t *e = l == 0 && prof ? prof->begin(bytes) : nullptr;
     if (e)
         hipExtLaunchKernelGGL(k, dim3(blocks), dim3(kMarchThreads), 0, s, e[0], e[1], 0, L.k(), g, L.g, b,
-                              (const T *)L.x, (const T *)C.x, L.xt, (T *)nullptr, dot, (const double *)nullptr);
+                              (const T *)L.x, (const T *)C.x, L.xt, (T *)nullptr, dot, StopK{});
     else
-        k<<<blocks, kMarchThreads, 0, s>>>(L.k(), g, L.g, b, L.x, C.x, L.xt, nullptr, dot, nullptr);
+        k<<<blocks, kMarchThreads, 0, s>>>(L.k(), g, L.g, b, L.x, C.x, L.xt, nullptr, dot, StopK{});
     std::swap(L.x, L.xt);
     return blocks;
 }
 
 // The start of a V-cycle on the finest level, queued ahead by the outer
 // iteration: its pre-leg, or else its first pre-sweep (which swaps the
-// iterate buffers); returns at once when *skip is non-zero.
+// iterate buffers); returns at once when the iteration has stopped.
 template <class T>
-static void queue_first(Hier<T> &H, const T *fineb, const Cycle &cy, hipStream_t s, const double *skip) {
-    if (leg_ok(H.lv[0], cy)) leg_pre(H.lv[0], H.lv[1], fineb, cy, s, skip);
-    else if (march_ok(H.lv[0], cy)) march_pre(H.lv[0], H.lv[1], fineb, cy, s, skip);
-    else rb_sweep<T>(H.lv[0], 0, fineb, 0, true, cy, nullptr, s, nullptr, nullptr, skip);
+static void queue_first(Hier<T> &H, const T *fineb, const Cycle &cy, hipStream_t s, const StopK &stop) {
+    if (leg_ok(H.lv[0], cy)) leg_pre(H.lv[0], H.lv[1], fineb, cy, s, stop);
+    else if (march_ok(H.lv[0], cy)) march_pre(H.lv[0], H.lv[1], fineb, cy, s, stop);
+    else rb_sweep<T>(H.lv[0], 0, fineb, 0, true, cy, nullptr, s, nullptr, nullptr, stop.skip);
+}
+// Most partials of r.r that the queued kernel sums itself (the one-region
+// legs only).
+template <class T>
+static int fold_rr(const Hier<T> &H, const Cycle &cy) {
+    return leg_ok(H.lv[0], cy) ? kFoldParts : 0;
 }
 // Whether the look-ahead applies: the finest level runs legs or fused sweeps
 // and the cycle has a level below it.
@@ -3245,8 +3235,8 @@ static int fast_setup(pps_handle *h, const double *dA, const double *dp, bool mi
                                                           V.x, V.r, f32, r32, part, flags, wx, wy, wz);
     }
     // deferred: r.r, b.b and the flags go to the mailbox as well
-    if (defer) k_scal_rr<<<1, 1024, 0, s>>>(part, zg.blocks, 1, S, h->mbox, ++h->mseq, flags);
-    else k_scal_rr<<<1, 1024, 0, s>>>(part, zg.blocks, 1, S);
+    if (defer) k_scal_rr<<<1, 1024, 0, s>>>(part, zg.blocks, 1, S, 1, h->mbox, ++h->mseq, flags);
+    else k_scal_rr<<<1, 1024, 0, s>>>(part, zg.blocks, 1, S, 1);
     PPS_HIP(hipGetLastError());
     // the hierarchy of the chosen precision, built on stream st
     auto build = [&](int singular, hipStream_t st) -> int {
@@ -3324,10 +3314,9 @@ static int outer_iterate(pps_handle *h, Hier<T> &H, bool mixed, double tol_abs, 
     if (!f->have_r) {
         if (f->exact) k_outer_resid<float, true><<<zg.grid, zb, 0, s>>>(O, zg.zc, V.b, V.x, V.r, b32, part);
         else k_outer_resid<float, false><<<zg.grid, zb, 0, s>>>(O, zg.zc, V.b, V.x, V.r, b32, part);
-        k_scal_rr<<<1, 1024, 0, s>>>(part, zg.blocks, 1, S, h->mbox, ++h->mseq);
+        k_scal_rr<<<1, 1024, 0, s>>>(part, zg.blocks, 1, S, 1, h->mbox, ++h->mseq);
     }
     f->have_r = 0;
-    k_outer_start<<<1, 64, 0, s>>>(S);
     PPS_HIP(hipGetLastError());
     // r.r of the setup pass or of the residual above
     PPS_TRY(wait_mailbox(h, s));
@@ -3404,6 +3393,7 @@ static int outer_iterate(pps_handle *h, Hier<T> &H, bool mixed, double tol_abs, 
     const bool ahead = can_queue_first(H, cy);
     bool queued = false;
     for (k = 1; k <= maxit; ++k) {
+        int nrr = 0;   // partials of r.r
         // z = V(r)
         const int ndot = vcycle<T>(H, fb, cy, &h->prof, s, cg ? part : nullptr,
                                    f->coarse_pending ? h->sev[1] : nullptr, queued);
@@ -3418,30 +3408,41 @@ static int outer_iterate(pps_handle *h, Hier<T> &H, bool mixed, double tol_abs, 
                 k_dot_rz<T><<<nb, 256, 0, s>>>(n, V.r, z, part);
                 nbz = nb;
             }
-            k_scal_beta<<<1, 1024, 0, s>>>(part, nbz, n, f->singular, S);
+            // few partials: the blocks of k_dq_tiled and k_update sum them
+            // (nb), many: a kernel of one workgroup does
+            const BetaK bk{nbz, f->singular, k == 1, S_RZ + ((k - 1) & 1), S_RZ + (k & 1), n};
+            AlphaK ak{tg.blocks, S_RZ + (k & 1), k % R};
+            const bool fold = nbz <= kFoldParts;
+            if (!fold) k_scal_beta<<<1, 1024, 0, s>>>(part, bk, S);
             // d_k's slot holds d_(k-R): applied first when still pending
             if (lazy && k - p0 >= R) flush(k - 1);
             T *dold = dslot(k - 1), *dnew = dslot(k);
             double *xu = lazy ? nullptr : V.x;
-            if (f->exact)
-                k_dq_tiled<T, true><<<tg.blocks, dim3(64, 16, 1), 0, s>>>(O, tg, z, dold, dnew, V.q, xu, S,
-                                                                          part);
-            else
-                k_dq_tiled<T, false><<<tg.blocks, dim3(64, 16, 1), 0, s>>>(O, tg, z, dold, dnew, V.q, xu, S,
-                                                                           part);
+            auto kdq = f->exact ? (fold ? k_dq_tiled<T, true, true> : k_dq_tiled<T, true, false>)
+                                : (fold ? k_dq_tiled<T, false, true> : k_dq_tiled<T, false, false>);
+            kdq<<<tg.blocks, dim3(64, 16, 1), 0, s>>>(O, tg, z, dold, dnew, V.q, xu, S, part, bk);
             if (!lazy) p0 = k;   // d_(k-1) applied in k_dq_tiled
-            k_scal_alpha<<<1, 1024, 0, s>>>(part, tg.blocks, S, k % R);
-            k_update<float><<<nb, 256, 0, s>>>(n, V.r, V.q, b32, S, part);
-            k_scal_rr<<<1, 1024, 0, s>>>(part, nb, 0, S, h->mbox, ++h->mseq, nullptr, N, tol_abs);
+            if (tg.blocks > kFoldParts) {
+                k_scal_alpha<<<1, 1024, 0, s>>>(part, ak, S);
+                ak.nb = 0;
+            }
+            k_update<float><<<nb, 256, 0, s>>>(n, V.r, V.q, b32, S, part, ak);
+            nrr = nb;
         } else {
             k_zsum<T><<<nb, 256, 0, s>>>(n, z, part);
             k_add_z<T><<<nb, 256, 0, s>>>(n, V.x, z, part, nb, f->singular);
             if (f->exact) k_outer_resid<float, true><<<zg.grid, zb, 0, s>>>(O, zg.zc, V.b, V.x, V.r, b32, part);
             else k_outer_resid<float, false><<<zg.grid, zb, 0, s>>>(O, zg.zc, V.b, V.x, V.r, b32, part);
-            k_scal_rr<<<1, 1024, 0, s>>>(part, zg.blocks, 0, S, h->mbox, ++h->mseq, nullptr, N, tol_abs);
+            nrr = zg.blocks;
         }
+        // r.r, the stopping test and the host's copy: in the queued leg's
+        // blocks where they are few, else in a kernel of their own before it
+        const StopK sk{S + S_STOP, part, ahead && k < maxit && nrr <= fold_rr(H, cy) ? nrr : 0, N, tol_abs, S,
+                       h->mbox, ++h->mseq};
+        if (!sk.nb)
+            k_scal_rr<<<1, 1024, 0, s>>>(part, nrr, 0, S, 0, h->mbox, h->mseq, nullptr, N, tol_abs);
         if (ahead && k < maxit) {
-            queue_first(H, fb, cy, s, S + S_STOP);
+            queue_first(H, fb, cy, s, sk);
             queued = true;
         }
         PPS_HIP(hipGetLastError());
@@ -3545,7 +3546,7 @@ int fast_solve(pps_handle *h, const double *dA, double *dp, double maxError, int
                                            wy, wz, s);
             else launch_check<double>(f, d, tg, (const double *)pend, S, dp, part, proj != nullptr, P, wx, wy,
                                       wz, s);
-            k_scal_rr<<<1, 1024, 0, s>>>(part, tg.blocks, 0, S);
+            k_scal_rr<<<1, 1024, 0, s>>>(part, tg.blocks, 0, S, 0);
             PPS_HIP(hipGetLastError());
             PPS_HIP(hipMemcpyAsync(h->pinned, S + S_RR, sizeof(double), hipMemcpyDeviceToHost, s));
             PPS_HIP(hipStreamSynchronize(s));
@@ -3623,7 +3624,7 @@ int fast_adjoint(pps_handle *h, const double *dA, const double *dg, double *dlam
     const int nbr = nblk(n);
     float *b32 = mixed ? f->b32.as<float>() : nullptr;
     k_resid_zero<float><<<nbr, 256, 0, s>>>(n, V.b, V.r, b32, part);
-    k_scal_rr<<<1, 1024, 0, s>>>(part, nbr, 1, S, h->mbox, ++h->mseq);
+    k_scal_rr<<<1, 1024, 0, s>>>(part, nbr, 1, S, 1, h->mbox, ++h->mseq);
     PPS_HIP(hipGetLastError());
     PPS_TRY(wait_mailbox(h, s));
     const double gg = h->mbox->bb;

@@ -25,6 +25,7 @@
 // second cell of an odd row's last pair.
 #pragma once
 
+#include "pps_scal.h"
 #include "pps_tail.h"
 #include "pps_xcd.h"
 
@@ -245,12 +246,12 @@ __device__ __forceinline__ void leg_tile(const LegK &g, int oz_cells, int &ox, i
 }
 
 // xo = two sweeps (colour 0 first) from zero for the right-hand side b, and
-// bc = the restricted residual.  skip: as in k_rb_sweep.
+// bc = the restricted residual.  Nothing once the outer iteration has stopped.
 template <class T, bool DGI, int EZ>
 __global__ void __launch_bounds__(kLegThreads)
 k_leg_pre(LevelK<T> L, LegK g, Coarsening cg, const T *__restrict__ b, T *__restrict__ xo, T *__restrict__ bc,
-          const double *__restrict__ skip) {
-    if (skip && *skip != 0.0) return;
+          StopK stop) {
+    if (stopped(stop)) return;
     using Lg = Leg<T, DGI, EZ>;
     __shared__ typename Lg::Lds lds;
     int ox, oy, oz;

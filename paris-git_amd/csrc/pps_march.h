@@ -41,6 +41,7 @@
 #pragma once
 
 #include "pps_leg.h"
+#include "pps_scal.h"
 #include "pps_tail.h"
 #include "pps_xcd.h"
 
@@ -107,8 +108,8 @@ template <class T, bool PRE, bool DOT, bool V16>
 __global__ void __launch_bounds__(kMarchThreads, sizeof(T) == 4 ? 4 : 2)
 k_march(LevelK<T> L, MarchK g, Coarsening cg, const T *__restrict__ b, const T *__restrict__ xc,
         const T *__restrict__ ec, T *__restrict__ xo, T *__restrict__ bc, double *__restrict__ part,
-        const double *__restrict__ skip) {
-    if (PRE && skip && *skip != 0.0) return;
+        StopK stop) {
+    if (PRE && stopped(stop)) return;
     using Pl = MarchPlane<T, PRE>;
     // three planes, distinct arrays (so that the compiler can tell a read of
     // one from the loads into another)
