@@ -2845,10 +2845,10 @@ static int leg_post(Level<T> &L, int l, const Level<T> &C, const T *b, const Cyc
 }
 
 // Whether level l's legs march (k_march): the default cycle on the larger
-// levels of a singular system.  256^3 FP32: 111 + 142 us against 198 + 162
-// for the sweeps and the restriction (FP64 169 + 218 against 484 + 409);
-// 128^3 FP32 23 + 25 against 42 + 38, FP64 39 + 36 against 82 + 54; 100^3
-// FP32 20 + 20 against 32 + 38.  64^3 FP64 16.5 + 18 against 17.5 + 21 for
+// levels of a singular system.  256^3 FP32: 89 + 116 us against 198 + 162
+// for the sweeps and the restriction (FP64 164 + 206 against 484 + 409);
+// 128^3 FP32 23 + 25 against 42 + 38, FP64 36 + 30 against 82 + 54; 100^3
+// FP32 20 + 20 against 32 + 38.  64^3 FP64 16.5 + 15 against 17.5 + 21 for
 // the one-region legs; 64^3 FP32 15 + 13 against their 9.1 + 9.3.
 template <class T>
 static bool march_ok(const Level<T> &L, const Cycle &cy) {
@@ -2856,12 +2856,12 @@ static bool march_ok(const Level<T> &L, const Cycle &cy) {
            L.n > kLegCells<T> && L.n * (long long)sizeof(T) < (1LL << 32) && L.nx >= 16 && L.ny >= 16 && L.nz >= 8;
 }
 // Blocks of a marching leg: the planes of a block that minimise rounds of
-// blocks (two fit a CU in FP32, one in FP64) x steps of a block.
+// blocks (one fits a CU) x steps of a block.
 template <class T>
 static MarchK march_grid(const Level<T> &L, const Cycle &cy, int *blocks) {
-    MarchK g{cy.per[0], cy.per[1], cy.per[2], (L.nx + kMarchOut - 1) / kMarchOut, (L.ny + kMarchOut - 1) / kMarchOut, 2};
+    MarchK g{cy.per[0], cy.per[1], cy.per[2], (L.nx + kMarchOutX<T> - 1) / kMarchOutX<T>, (L.ny + kMarchOut - 1) / kMarchOut, 2};
     const long long cols = (long long)g.tx * g.ty;
-    const int slots = cy.cus * (sizeof(T) == 4 ? 2 : 1);
+    const int slots = cy.cus;
     long long best = -1;
     for (int zc = 2; zc <= ((L.nz + 1) & ~1); zc += 2) {
         const long long nb = cols * ((L.nz + zc - 1) / zc);
@@ -2877,7 +2877,7 @@ static void march_pre(const Level<T> &L, const Level<T> &C, const T *b, const Cy
     int blocks;
     const MarchK g = march_grid(L, cy, &blocks);
     auto k = L.nx % (16 / (int)sizeof(T)) == 0 ? k_march<T, true, false, true> : k_march<T, true, false, false>;
-    k<<<blocks, kMarchThreads, 0, s>>>(L.k(), g, L.g, b, nullptr, nullptr, L.x, C.b, nullptr, stop);
+    k<<<blocks, kMarchThreads<T>, 0, s>>>(L.k(), g, L.g, b, nullptr, nullptr, L.x, C.b, nullptr, stop);
 }
 template <class T>
 static int march_post(Level<T> &L, int l, const Level<T> &C, const T *b, const Cycle &cy, Prof *prof, hipStream_t s,
@@ -2892,10 +2892,10 @@ static int march_post(Level<T> &L, int l, const Level<T> &C, const T *b, const C
     const double bytes = (double)sizeof(T) * ((double)L.n * 5.5 + (double)C.n);
     hipEvent_t *e = l == 0 && prof ? prof->begin(bytes) : nullptr;
     if (e)
-        hipExtLaunchKernelGGL(k, dim3(blocks), dim3(kMarchThreads), 0, s, e[0], e[1], 0, L.k(), g, L.g, b,
+        hipExtLaunchKernelGGL(k, dim3(blocks), dim3(kMarchThreads<T>), 0, s, e[0], e[1], 0, L.k(), g, L.g, b,
                               (const T *)L.x, (const T *)C.x, L.xt, (T *)nullptr, dot, StopK{});
     else
-        k<<<blocks, kMarchThreads, 0, s>>>(L.k(), g, L.g, b, L.x, C.x, L.xt, nullptr, dot, StopK{});
+        k<<<blocks, kMarchThreads<T>, 0, s>>>(L.k(), g, L.g, b, L.x, C.x, L.xt, nullptr, dot, StopK{});
     std::swap(L.x, L.xt);
     return blocks;
 }

@@ -4,24 +4,32 @@
 // iterate is zero, and after them the residual is restricted (PRE); or the
 // coarse correction is added before them (POST).  Sweep by sweep the level's
 // couplings, right-hand side and iterate stream from HBM two or three times.
-// Here a block marches the planes of a 32 x 32 region once, its four colour
-// passes (and the residual) trailing each other by one plane:
+// Here a block marches the planes of a region of 64 x 32 cells (FP64 32 x 32)
+// once, its four colour passes (and the residual) trailing each other by one plane:
 //   step s:  plane s    rows and right-hand side, first values of colour 0
 //            plane s-1  colour 1
 //            plane s-2  colour 0
 //            plane s-3  colour 1
 //            plane s-4  colour 0 (POST) or its residual (PRE); output
 // Each pass is right one cell further inside than the one before, so the
-// inner 24 x 24 cells are those of the sweeps on the whole level; the halo
-// is computed 1.8 times over and read again from the L2, where neighbouring
-// tiles (numbered XCD by XCD) find each other's lines.
+// inner 56 x 24 cells (FP64 24 x 24) are those of the sweeps on the whole
+// level; cells are computed 1.5 times over (FP64 1.8) and the halo read again
+// from the L2, where neighbouring tiles (numbered XCD by XCD) find each
+// other's lines if they march at one pace.  So a block fills a CU: of two
+// 512-thread blocks (32 x 32 in FP32 too) one was served first and ran up to
+// 30 planes ahead, and its lines had gone when the other came: 389 and 534 MB
+// fetched at 256^3 (PRE, POST; least 268 and 310) instead of 332 and 429.
 //
 // Planes are loaded straight into LDS (buffer loads with an LDS target, two
 // planes ahead: no registers are held by loads in flight, and a load's
-// latency spans two steps).  A thread owns the column of one x-pair (2m,
+// latency spans two steps).  Rows of one parity issue them at the start of a
+// step and the others at its end, so that half of the wavefronts compute
+// while the other half waits for the load unit (256^3 FP32 94 + 122 us with
+// all at the start, 89 + 116 so).  A thread owns the column of one x-pair (2m,
 // 2m+1) of one row: the rows of its last planes and all vertical neighbours
-// are in its registers; in-plane neighbours come from LDS, where each stage
-// leaves the value it formed for the stage behind it, one step later.  A
+// are in its registers, neighbours along x in the next lanes'; those along y
+// come from LDS, where each stage leaves the value it formed for the stage
+// behind it, one step later.  A
 // stage reads only what earlier steps wrote: one barrier a step.
 // j + k has one parity over a wavefront, so the position in the pair that
 // all stages of a step update is the same and uniform; the steps are
@@ -47,9 +55,11 @@
 
 namespace pps {
 
-constexpr int kMarchOut = 24;            // output cells along x and y
-constexpr int kMarchThreads = 512;       // 16 pairs x 32 rows
 constexpr int kMarchHalo = 4;
+constexpr int kMarchOut = 24;                                       // output rows of a tile
+template <class T> constexpr int kMarchPairs = sizeof(T) == 4 ? 32 : 16;   // pairs of a row of a region
+template <class T> constexpr int kMarchOutX = 2 * kMarchPairs<T> - 2 * kMarchHalo;   // output cells of it
+template <class T> constexpr int kMarchThreads = 32 * kMarchPairs<T>;
 
 struct MarchK {
     int px, py, pz;      // periodic axes
@@ -81,9 +91,27 @@ template <class T> struct Buf {
     }
 };
 
-// s_waitcnt vmcnt(N) alone
+// Until at most N of the wavefront's loads and stores are outstanding (they
+// are counted in the order of their issue).
 template <int N> __device__ __forceinline__ void wait_vm() {
-    __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0f70);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+// v of the lane above (UP) or below: within rows of 16 lanes (R 16) or within
+// the wavefront; 0 beyond the end.
+template <bool UP, int R> __device__ __forceinline__ int beside(int v) {
+    constexpr int ctrl = R == 16 ? (UP ? 0x101 : 0x111) : (UP ? 0x130 : 0x138);   // row / wave shl, shr
+    return __builtin_amdgcn_update_dpp(0, v, ctrl, 0xf, 0xf, true);
+}
+template <bool UP, int R> __device__ __forceinline__ float beside(float v) {
+    return __builtin_bit_cast(float, beside<UP, R>(__builtin_bit_cast(int, v)));
+}
+template <bool UP, int R> __device__ __forceinline__ double beside(double v) {
+    union { double d; int i[2]; } u;
+    u.d = v;
+    u.i[0] = beside<UP, R>(u.i[0]);
+    u.i[1] = beside<UP, R>(u.i[1]);
+    return u.d;
 }
 
 // Workgroup barrier over LDS reads and writes.  lds_barrier's fence would
@@ -98,14 +126,15 @@ __device__ __forceinline__ void march_barrier() {
 // below it, POST the colour-0 iterate (one a pair) and the correction of it.
 template <class T> struct alignas(2 * sizeof(T)) LdsPair { T a, b; };   // one LDS access
 template <class T, bool PRE> struct alignas(16) MarchPlane {
-    LdsPair<T> cx[kMarchThreads], cy[kMarchThreads], cz[kMarchThreads], b[kMarchThreads];
-    T e0[PRE ? 32 : kMarchThreads], e1[PRE ? 32 : kMarchThreads];
+    static constexpr int N = kMarchThreads<T>;
+    LdsPair<T> cx[N], cy[N], cz[N], b[N];
+    T e0[PRE ? 32 : N], e1[PRE ? 2 * kMarchPairs<T> : N];
 };
 
 // V16: rows are multiples of 16 bytes, and planes are loaded 16 bytes a lane
 // (a wavefront half an array); otherwise 4 bytes a lane, any row length.
 template <class T, bool PRE, bool DOT, bool V16>
-__global__ void __launch_bounds__(kMarchThreads, sizeof(T) == 4 ? 4 : 2)
+__global__ void __launch_bounds__(kMarchThreads<T>, sizeof(T) == 4 ? 4 : 2)
 k_march(LevelK<T> L, MarchK g, Coarsening cg, const T *__restrict__ b, const T *__restrict__ xc,
         const T *__restrict__ ec, T *__restrict__ xo, T *__restrict__ bc, double *__restrict__ part,
         StopK stop) {
@@ -115,15 +144,15 @@ k_march(LevelK<T> L, MarchK g, Coarsening cg, const T *__restrict__ b, const T *
     // one from the loads into another)
     __shared__ Pl A0, A1, A2;
     // what each stage formed in the last two steps, one a pair, and PRE's
-    // residuals; a padding value at both ends for the edge pairs' reads
-    constexpr int kW = kMarchThreads;
-    __shared__ T Wm[4 * 2 * kW + 2];
+    // residuals
+    constexpr int kW = kMarchThreads<T>, kR = kMarchPairs<T>, kC = 2 * kR;   // pairs, pairs and cells of a row
+    __shared__ T Wm[4 * 2 * kW];
     __shared__ T Rz[PRE ? 2 * kW : 1];
     const int nx = L.nx, ny = L.ny, nz = L.nz;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int t = xcd_order(blockIdx.x, gridDim.x);
-    const int ox = t % g.tx * kMarchOut, oy = t / g.tx % g.ty * kMarchOut;
+    const int ox = t % g.tx * kMarchOutX<T>, oy = t / g.tx % g.ty * kMarchOut;
     const int k0 = t / (g.tx * g.ty) * g.zc, k1 = min(k0 + g.zc, (nz + 1) & ~1);
     auto place = [](int i, int n, int per) {   // wrapped, or moved to the nearest cell
         if (i >= 0 && i < n) return i;
@@ -134,52 +163,52 @@ k_march(LevelK<T> L, MarchK g, Coarsening cg, const T *__restrict__ b, const T *
     // the row of the region that lies at place r of a plane in LDS
     auto row_at = [](int r) { return 2 * (r & 15) + (r >> 4); };
 
-    // the thread's pair: 16 pairs x 4 rows of one parity jl a wavefront
-    const int m = tid & 15, jl = wv & 1, jh = (lane >> 4) + (wv >> 1) * 4, j = 2 * jh + jl;
-    const int own = m + 16 * jh + 256 * jl;
-    const int rs = own + (jl ? -256 : 240), rn = own + (jl ? -240 : 256);   // rows below, above
+    // the thread's pair: the pairs of 64 / kR rows of one parity jl a wavefront
+    const int m = tid & (kR - 1), jl = wv & 1, jh = lane / kR + (wv >> 1) * (64 / kR), j = 2 * jh + jl;
+    const int own = m + kR * jh + kW / 2 * jl;
+    const int rs = own + (jl ? -kW / 2 : kW / 2 - kR), rn = own + (jl ? kR - kW / 2 : kW / 2);   // rows below, above
     const int ui = ox - kMarchHalo + 2 * m, uj = oy - kMarchHalo + j;
     const int gi = place(ui, nx, g.px) & ~1, gj = place(uj, ny, g.py);
-    const bool two = gi + 1 < nx;            // the pair's second cell exists
-    const bool mine = m >= 2 && m < 14 && j >= 4 && j < 28 && ui < nx && uj < ny;
+    const bool two = V16 || gi + 1 < nx;     // the pair's second cell exists
+    const bool mine = m >= 2 && m < kR - 2 && j >= 4 && j < 28 && ui < nx && uj < ny;
     const bool wallw = ui == 0 && !g.px, walls = uj == 0 && !g.py;   // no coupling to the left, below
     const long long sz = (long long)nx * ny, n = sz * nz;
     const unsigned np = (nx + 1) >> 1, pcol = (gi >> 1) + np * gj;
     const long long psz = (long long)np * ny;
 
     // loads of a plane's four arrays, NC a wavefront (V16: of its own array
-    // wv / 2, else of each), and the lane's byte offsets in a plane
+    // wv / (kR / 8), else of each), and the lane's byte offsets in a plane
     constexpr int DW = sizeof(T) / 4, NC = 2 * DW;
     unsigned off[NC], pof[DW], eof[DW], off_w = 0, off_s = 0;
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
         // cell of the plane in LDS; V16: the first of the lane's 4 / DW cells,
         // all inside the row or all outside
-        const int e = V16 ? (((wv & 1) * NC + c) * 64 + lane) * (4 / DW) : ((wv * NC + c) * 64 + lane) / DW;
-        int i = place(ox - kMarchHalo + (e & 31), nx, g.px);
+        const int e = V16 ? (((wv & (kR / 8 - 1)) * NC + c) * 64 + lane) * (4 / DW) : ((wv * NC + c) * 64 + lane) / DW;
+        int i = place(ox - kMarchHalo + (e & (kC - 1)), nx, g.px);
         if (V16) i &= ~(4 / DW - 1);
-        off[c] = (i + (unsigned)nx * place(oy - kMarchHalo + row_at(e >> 5), ny, g.py)) * (unsigned)sizeof(T) +
+        off[c] = (i + (unsigned)nx * place(oy - kMarchHalo + row_at(e / kC), ny, g.py)) * (unsigned)sizeof(T) +
                  (V16 ? 0u : (lane % DW) * 4u);
     }
     if (PRE) {
-        const int e = lane / DW;   // 32 rows, 32 cells
+        const int e = lane / DW;   // 32 rows, kC cells
         off_w = (place(ox - kMarchHalo - 1, nx, g.px) +
                  (unsigned)nx * place(oy - kMarchHalo + row_at(e & 31), ny, g.py)) * (unsigned)sizeof(T) + (lane % DW) * 4u;
-        off_s = (place(ox - kMarchHalo + (e & 31), nx, g.px) +
+        off_s = (place(ox - kMarchHalo + (e & (kC - 1)), nx, g.px) +
                  (unsigned)nx * place(oy - kMarchHalo - 1, ny, g.py)) * (unsigned)sizeof(T) + (lane % DW) * 4u;
     } else {
-        // the wavefront's own 64 pairs (16 a row); the second cell's parent
+        // the wavefront's own 64 pairs; the second cell's parent
         // where cells and not pairs are children (fx 1) is the next element
 #pragma unroll
         for (int c = 0; c < DW; ++c) {
-            const int e = (c * 64 + lane) / DW, em = e & 15, ej = 2 * ((e >> 4) + (wv >> 1) * 4) + jl;
+            const int e = (c * 64 + lane) / DW, em = e & (kR - 1), ej = 2 * (e / kR + (wv >> 1) * (64 / kR)) + jl;
             const int i = place(ox - kMarchHalo + 2 * em, nx, g.px) & ~1, jj = place(oy - kMarchHalo + ej, ny, g.py);
             pof[c] = ((i >> 1) + np * jj) * (unsigned)sizeof(T) + (lane % DW) * 4u;
             eof[c] = ((i >> (cg.fx - 1)) + (unsigned)cg.cnx * (jj >> (cg.fy - 1))) * (unsigned)sizeof(T) + (lane % DW) * 4u;
         }
     }
     const Buf<T> Bx(L.cx, n), By(L.cy, n), Bz(L.cz, n), Bb(b, n);
-    const Buf<T> Bm(wv < 2 ? L.cx : wv < 4 ? L.cy : wv < 6 ? L.cz : b, n);   // V16: this wavefront's array
+    const Buf<T> Bm(wv < kR / 8 ? L.cx : wv < kR / 4 ? L.cy : wv < 3 * kR / 8 ? L.cz : b, n);   // V16: this wavefront's array
     const Buf<T> Bc(PRE ? b : xc, PRE ? n : psz * nz);
     const Buf<T> Be(PRE ? b : ec, PRE ? n : (long long)cg.cnx * cg.cny * cg.cnz);
     auto plane_of = [&](int k) {   // wrapped; -1 beyond a wall (uniform)
@@ -208,24 +237,25 @@ k_march(LevelK<T> L, MarchK g, Coarsening cg, const T *__restrict__ b, const T *
             }
         }
         if (PRE) {
-            if (lane < 32 * DW) {
-                if (wv == 0) Bx.template to_lds<4>(A.e0, o, off_w);
-                if (wv == 1) By.template to_lds<4>(A.e1, o, off_s);
-            }
+            if (wv == 0 && lane < 32 * DW) Bx.template to_lds<4>(A.e0, o, off_w);
+            if (wv == 1 && lane < kC * DW) By.template to_lds<4>(A.e1, o, off_s);
         } else {
             const unsigned ko = (unsigned)(cg.cnx * cg.cny) * (k >> (cg.fz - 1)) + (cg.fx == 1 ? e : 0);
 #pragma unroll
             for (int c = 0; c < DW; ++c) {
-                const int d = 64 * (wv >> 1) + 256 * jl + c * 64 / DW;
+                const int d = 64 * (wv >> 1) + kW / 2 * jl + c * 64 / DW;
                 Bc.template to_lds<4>(A.e0 + d, (unsigned)psz * k, pof[c]);
                 Be.template to_lds<4>(A.e1 + d, ko, eof[c]);
             }
         }
         return true;
     };
-    // a plane's loads at least (the count of every wavefront): waiting until
-    // no more are outstanding than were issued for the plane behind it means
-    // that its own have landed (stores in between make the wait stricter)
+    // A plane's loads at least (the count of every wavefront).  A step waits
+    // until nothing older than what it and the step before issued since is
+    // outstanding: its loads for plane s + 2 and both steps' stores, which
+    // stay in flight (to wait for one of those loads costs a memory latency a
+    // step: 256^3 FP32 PRE 99 us, POST 135; counted 95 and 124).  A count too
+    // low is safe.
     constexpr int kLoads = (V16 ? 1 : 4) * NC + (PRE ? 0 : 2 * DW);
 
     // rows of the last planes by position, and the values of both colours in
@@ -238,8 +268,12 @@ k_march(LevelK<T> L, MarchK g, Coarsening cg, const T *__restrict__ b, const T *
 #pragma unroll
         for (int e = 0; e < 2; ++e) cx[q][e] = cs[q][e] = cn[q][e] = cu[q][e] = bb[q][e] = rd[q][e] = (T)0;
     }
-    for (int e = tid; e < 4 * 2 * kW + 2; e += kMarchThreads) Wm[e] = (T)0;
+    for (int e = tid; e < 4 * 2 * kW; e += kW) Wm[e] = (T)0;
     double sbx = 0.0, sx = 0.0, sb = 0.0;
+    // whether the wavefront stores (a value a step), and how often in two
+    // steps it stores a restricted one (PRE)
+    const bool storing = __any(mine);
+    const int bstores = !PRE || (cg.fy == 2 && jl) ? 0 : cg.fz == 2 ? 1 : 2;
 
     // restriction of plane k, whose residuals were formed in the step before
     // (rlast, and the next row's in LDS); e: position of colour 0 in this
@@ -249,7 +283,7 @@ k_march(LevelK<T> L, MarchK g, Coarsening cg, const T *__restrict__ b, const T *
     T rlast = 0, rsum[2] = {0, 0};
     auto finish = [&](int k, int e) {
         if (cg.fy == 2 && jl) return;   // uniform
-        const T r2 = cg.fy == 2 ? Rz[(k & 1) * kW + own + 256] : (T)0;
+        const T r2 = cg.fy == 2 ? Rz[(k & 1) * kW + own + kW / 2] : (T)0;
         T va = e ? r2 : rlast, vb = e ? rlast : r2;
         if (cg.fz == 2 && !(k & 1)) {
             rsum[0] = va;
@@ -269,14 +303,15 @@ k_march(LevelK<T> L, MarchK g, Coarsening cg, const T *__restrict__ b, const T *
         }
     };
 
-    // step s at place P0 of the register rings, the active position E, the
+    // step s at place P0 of the register rings, LATE: requests last, the active position E, the
     // plane in A, and An the LDS to load plane s + 2 into
-    auto step = [&](auto PC, auto EC, Pl &A, Pl &An, int s) {
+    auto step = [&](auto LC, auto PC, auto EC, Pl &A, Pl &An, int s) {
+        constexpr bool LATE = decltype(LC)::value;
         constexpr int P0 = decltype(PC)::value, E = decltype(EC)::value, H = P0 & 1;
         constexpr int P1 = (P0 + 5) % 6, P2 = (P0 + 4) % 6, P3 = (P0 + 3) % 6, P4 = (P0 + 2) % 6;
         // a stage's output of this step, and of the step before
-        auto W = [&](int st, int i) -> T & { return Wm[1 + (st * 2 + H) * kW + i]; };
-        auto V = [&](int st, int i) -> T { return Wm[1 + (st * 2 + 1 - H) * kW + i]; };
+        auto W = [&](int st, int i) -> T & { return Wm[(st * 2 + H) * kW + i]; };
+        auto V = [&](int st, int i) -> T { return Wm[(st * 2 + 1 - H) * kW + i]; };
         // b + sum of the couplings of the cell at position E of plane slot q,
         // the neighbours of stage st; xp its pair's other cell, xd / xu the
         // cells below and above, cd the coupling to the one below (the +z
@@ -284,19 +319,20 @@ k_march(LevelK<T> L, MarchK g, Coarsening cg, const T *__restrict__ b, const T *
         auto sum = [&](auto QC, int st, T xp, T cd, T xd, T xu) {
             constexpr int q = decltype(QC)::value;
             T v = bb[q][E] + co[q] * xp;
-            v += cx[q][E] * V(st, own + (E ? 1 : -1));
+            v += cx[q][E] * beside<E == 1, kR>(xp);   // the same stage's value of the next pair
             v += cs[q][E] * V(st, rs);
             v += cn[q][E] * V(st, rn);
             v += cd * xd;
             v += cu[q][E] * xu;
             return v;
         };
-        const bool ahead = request(An, s + 2, E);
+        bool ahead = false;
+        if (!LATE) ahead = request(An, s + 2, E);
         if (PRE && s - 5 >= k0) finish(s - 5, 1 - E);
         // plane s
         if (plane_of(s) >= 0) {
             const LdsPair<T> vx = A.cx[own], vn = A.cy[own], vs = A.cy[rs], vu = A.cz[own], vb = A.b[own];
-            T left = lane_below(vx.b);
+            T left = beside<false, kR>(vx.b);
             if (PRE) left = m == 0 ? A.e0[jh + 16 * jl] : left;
             co[P0] = vx.a;
             cx[P0][0] = wallw ? (T)0 : left;
@@ -349,9 +385,14 @@ k_march(LevelK<T> L, MarchK g, Coarsening cg, const T *__restrict__ b, const T *
                 }
             }
         }
+        if (LATE) ahead = request(An, s + 2, E);
         // plane s + 1 (requested a step ago) has landed
-        if (ahead) wait_vm<kLoads>();
-        else wait_vm<0>();
+        if (!ahead) wait_vm<0>();
+        else if (!(storing && k - (PRE ? 2 : 1) >= k0 && k < nz)) wait_vm<kLoads>();
+        else if (LATE) wait_vm<kLoads + 1>();
+        else if (bstores == 0) wait_vm<kLoads + 2>();
+        else if (bstores == 1) wait_vm<kLoads + 3>();
+        else wait_vm<kLoads + 4>();
         march_barrier();
         __builtin_amdgcn_sched_barrier(0);   // nothing of the next step moves up (registers)
     };
@@ -374,14 +415,14 @@ k_march(LevelK<T> L, MarchK g, Coarsening cg, const T *__restrict__ b, const T *
     auto run = [&](auto EC) {
         constexpr int E = decltype(EC)::value;
         for (int s = s0;; s += 6) {
-            step(Ic<0>(), Ic<E>(), A0, A2, s);
-            step(Ic<1>(), Ic<1 - E>(), A1, A0, s + 1);
+            step(EC, Ic<0>(), Ic<E>(), A0, A2, s);
+            step(EC, Ic<1>(), Ic<1 - E>(), A1, A0, s + 1);
             if (s + 2 > s1) break;
-            step(Ic<2>(), Ic<E>(), A2, A1, s + 2);
-            step(Ic<3>(), Ic<1 - E>(), A0, A2, s + 3);
+            step(EC, Ic<2>(), Ic<E>(), A2, A1, s + 2);
+            step(EC, Ic<3>(), Ic<1 - E>(), A0, A2, s + 3);
             if (s + 4 > s1) break;
-            step(Ic<4>(), Ic<E>(), A1, A0, s + 4);
-            step(Ic<5>(), Ic<1 - E>(), A2, A1, s + 5);
+            step(EC, Ic<4>(), Ic<E>(), A1, A0, s + 4);
+            step(EC, Ic<5>(), Ic<1 - E>(), A2, A1, s + 5);
             if (s + 6 > s1) break;
         }
     };
