@@ -1565,8 +1565,9 @@ k_dq_tiled(OpK L, TGrid g, const TZ *__restrict__ z, const TZ *__restrict__ dold
     double beta, zm;
     if constexpr (FOLD) {
         double sums[3], rho;
+        const double rho_old = S[bk.rd];
         sum_partials3(part, bk.nb, sums);
-        beta_of(bk, sums, S, &beta, &zm, &rho);
+        beta_of(bk, sums, rho_old, &beta, &zm, &rho);
         beta = uniform(beta);
         zm = uniform(zm);
         if (blockIdx.x == 0 && threadIdx.x + threadIdx.y == 0) S[bk.wr] = rho;
@@ -1691,14 +1692,24 @@ k_update(long long n, double *__restrict__ r, const double *__restrict__ q, TB *
     } else {
         alpha = S[S_ALPHA];
     }
+    // (q starts at an odd element where n is odd: half the natural alignment)
+    using D2 = double __attribute__((ext_vector_type(2), aligned(8)));
+    using B2 = TB __attribute__((ext_vector_type(2), aligned(sizeof(TB))));
     double rr = 0.0;
-    for (long long c = blockIdx.x * 256LL + threadIdx.x; c < n; c += (long long)gridDim.x * 256) {
+    for (long long e = blockIdx.x * 256LL + threadIdx.x; e < n >> 1; e += (long long)gridDim.x * 256) {
         // r and q non-temporal; the FP32 copy of r, which the next V-cycle's
-        // first sweep reads at once, is cached (that sweep: 73.7 -> 63.8 us
-        // at 256^3)
-        const double v = __builtin_nontemporal_load(r + c) - alpha * __builtin_nontemporal_load(q + c);
-        __builtin_nontemporal_store(v, r + c);
-        if (bt) bt[c] = (TB)v;
+        // first leg reads at once, is cached
+        D2 v = __builtin_nontemporal_load(reinterpret_cast<const D2 *>(r) + e) -
+               alpha * __builtin_nontemporal_load(reinterpret_cast<const D2 *>(q) + e);
+        __builtin_nontemporal_store(v, reinterpret_cast<D2 *>(r) + e);
+        if (bt) reinterpret_cast<B2 *>(bt)[e] = __builtin_convertvector(v, B2);
+        rr += v.x * v.x;
+        rr += v.y * v.y;
+    }
+    if ((n & 1) && blockIdx.x == 0 && threadIdx.x == 0) {
+        const double v = r[n - 1] - alpha * q[n - 1];
+        r[n - 1] = v;
+        if (bt) bt[n - 1] = (TB)v;
         rr += v * v;
     }
     block_partial(rr, part);
@@ -1756,10 +1767,11 @@ k_add_z(long long n, double *__restrict__ x, const TZ *__restrict__ z, const dou
 __global__ void __launch_bounds__(1024)
 k_scal_beta(const double *__restrict__ part, BetaK bk, double *__restrict__ S) {
     double sums[3];
+    const double rho_old = S[bk.rd];   // in flight with the partials
     sum_partials3(part, bk.nb, sums);
     if (threadIdx.x == 0) {
         double beta, zm, rho;
-        beta_of(bk, sums, S, &beta, &zm, &rho);
+        beta_of(bk, sums, rho_old, &beta, &zm, &rho);
         S[S_BETA] = beta;
         S[bk.wr] = rho;
         S[S_ZMEAN] = zm;
@@ -1769,9 +1781,10 @@ k_scal_beta(const double *__restrict__ part, BetaK bk, double *__restrict__ S) {
 // the alpha step from k_dq_tiled's partials
 __global__ void __launch_bounds__(1024)
 k_scal_alpha(const double *__restrict__ part, AlphaK ak, double *__restrict__ S) {
+    const double rho = S[ak.rz];   // in flight with the partials
     const double dq = sum_partials(part + 3 * kRedBlocks, ak.nb);
     if (threadIdx.x == 0) {
-        const double alpha = S[ak.rz] / dq;
+        const double alpha = rho / dq;
         S[S_DQ] = dq;
         S[S_ALPHA] = alpha;
         S[S_AH + ak.slot] = alpha;
@@ -2351,13 +2364,21 @@ static dim3 cgrid3(int nx, int ny, int nz) {
 }
 static const dim3 kB3(64, 4, 1);
 // Blocks of the grid-stride streaming kernels (one partial each): 32 per CU
-// at most (k_update at 256^3: 81.3 us with 2048 blocks, 75.7 us with 8192;
-// the r.r kernel then sums 8192 partials, 6.3 -> 7.2 us).
+// at most.
 static int nblk(long long n) {
     long long b = (n + 255) / 256;
     if (b > 8192) b = 8192;
     if (b < 1) b = 1;
     return (int)b;
+}
+
+// k_update's, two cells a thread and turn: 128^3 12.8 us with 1024 blocks and
+// 12.9 with 4096 (15.9 with a cell a turn and 8192), 256^3 72 us with 1024
+// and 78 with 4096 (75); its 1024 partials are summed in 4.7 us (6.1 from
+// 8192).
+static int nblk_update(long long n) {
+    const long long b = (n / 2 + 255) / 256;
+    return (int)(b > 1024 ? 1024 : b < 1 ? 1 : b);
 }
 
 // Level sizes of the fast hierarchy.  From each level every axis is halved
@@ -3426,8 +3447,8 @@ static int outer_iterate(pps_handle *h, Hier<T> &H, bool mixed, double tol_abs, 
                 k_scal_alpha<<<1, 1024, 0, s>>>(part, ak, S);
                 ak.nb = 0;
             }
-            k_update<float><<<nb, 256, 0, s>>>(n, V.r, V.q, b32, S, part, ak);
-            nrr = nb;
+            nrr = nblk_update(n);
+            k_update<float><<<nrr, 256, 0, s>>>(n, V.r, V.q, b32, S, part, ak);
         } else {
             k_zsum<T><<<nb, 256, 0, s>>>(n, z, part);
             k_add_z<T><<<nb, 256, 0, s>>>(n, V.x, z, part, nb, f->singular);

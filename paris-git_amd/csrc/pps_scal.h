@@ -84,11 +84,11 @@ struct BetaK {
     int nb, singular, first, rd, wr;
     long long n;
 };
-__device__ __forceinline__ void beta_of(const BetaK &k, const double sums[3], const double *S, double *beta,
+__device__ __forceinline__ void beta_of(const BetaK &k, const double sums[3], double rho_old, double *beta,
                                         double *zm, double *rho) {
     *zm = k.singular ? sums[1] / (double)k.n : 0.0;
     *rho = sums[0] - *zm * sums[2];
-    *beta = k.first ? 0.0 : *rho / S[k.rd];
+    *beta = k.first ? 0.0 : *rho / rho_old;
 }
 
 // alpha = rho / d.q (nb 0: it is in S; rz: the place of rho; slot: the
