@@ -29,30 +29,38 @@ struct PairNb {
     int own, s, n, d, u, o[2];
 };
 
-// rows of pair m of row j, plane k
-template <class T, bool DGI>
-__device__ __forceinline__ void load_pair(const LevelK<T> &L, int m, int j, int k, PairRow<T> &P) {
-    const int sy = L.nx, sz = L.nx * L.ny, i = 2 * m;
-    const long long c = i + (long long)sy * j + (long long)sz * k;
-    const int o = i + 1 < L.nx ? 1 : 0;
-    const long long cw = m == 0 ? c + (L.nx - 1) : c - 1;
-    const long long cs = c + (long long)(wrap_m(j, L.ny) - j) * sy;
-    const long long cd = c + (long long)(wrap_m(k, L.nz) - k) * sz;
-    T xw = L.cx[cw], xa = L.cx[c], xb = L.cx[c + o];
-    T sa = L.cy[cs], sb = L.cy[cs + o], na = L.cy[c], nb = L.cy[c + o];
-    T da = L.cz[cd], db = L.cz[cd + o], ua = L.cz[c], ub = L.cz[c + o];
-    T ga = DGI ? diag_sum(xw, xa, sa, na, da, ua) : L.dg[c];
-    T gb = DGI ? diag_sum(xa, xb, sb, nb, db, ub) : L.dg[c + o];
-    if (!o) { xb = sb = nb = db = ub = (T)0; gb = (T)1; }
-    const bool e = (j + k) & 1;   // colour 0 is the pair's second cell
-    P.co = xa;
-    P.cxo[0] = e ? xb : xw; P.cxo[1] = e ? xw : xb;
-    P.cs[0] = e ? sb : sa; P.cs[1] = e ? sa : sb;
-    P.cn[0] = e ? nb : na; P.cn[1] = e ? na : nb;
-    P.cd[0] = e ? db : da; P.cd[1] = e ? da : db;
-    P.cu[0] = e ? ub : ua; P.cu[1] = e ? ua : ub;
-    P.rd[0] = (T)1 / (e ? gb : ga); P.rd[1] = (T)1 / (e ? ga : gb);
-}
+// What the rows of pair m of row j, plane k are formed from: loaded first for
+// all of a thread's pairs, so that one latency covers them.
+template <class T, bool DGI> struct PairLoad {
+    T xw, xa, xb, sa, sb, na, nb, da, db, ua, ub, ga, gb;
+    __device__ __forceinline__ void load(const LevelK<T> &L, int m, int j, int k) {
+        const int sy = L.nx, sz = L.nx * L.ny, i = 2 * m;
+        const long long c = i + (long long)sy * j + (long long)sz * k;
+        const int o = i + 1 < L.nx ? 1 : 0;
+        const long long cw = m == 0 ? c + (L.nx - 1) : c - 1;
+        const long long cs = c + (long long)(wrap_m(j, L.ny) - j) * sy;
+        const long long cd = c + (long long)(wrap_m(k, L.nz) - k) * sz;
+        xw = L.cx[cw], xa = L.cx[c], xb = L.cx[c + o];
+        sa = L.cy[cs], sb = L.cy[cs + o], na = L.cy[c], nb = L.cy[c + o];
+        da = L.cz[cd], db = L.cz[cd + o], ua = L.cz[c], ub = L.cz[c + o];
+        if (!DGI) { ga = L.dg[c]; gb = L.dg[c + o]; }
+    }
+    // o: the pair's second cell exists; e: colour 0 is that cell (j + k odd)
+    __device__ __forceinline__ void form(bool o, bool e, PairRow<T> &P) {
+        if (DGI) {
+            ga = diag_sum(xw, xa, sa, na, da, ua);
+            gb = diag_sum(xa, xb, sb, nb, db, ub);
+        }
+        if (!o) { xb = sb = nb = db = ub = (T)0; gb = (T)1; }
+        P.co = xa;
+        P.cxo[0] = e ? xb : xw; P.cxo[1] = e ? xw : xb;
+        P.cs[0] = e ? sb : sa; P.cs[1] = e ? sa : sb;
+        P.cn[0] = e ? nb : na; P.cn[1] = e ? na : nb;
+        P.cd[0] = e ? db : da; P.cd[1] = e ? da : db;
+        P.cu[0] = e ? ub : ua; P.cu[1] = e ? ua : ub;
+        P.rd[0] = (T)1 / (e ? gb : ga); P.rd[1] = (T)1 / (e ? ga : gb);
+    }
+};
 
 // b + sum coupling * neighbour of the pair's colour-Q cell: xo the pair's
 // other cell, O the other colour's LDS array
@@ -86,10 +94,11 @@ __device__ __forceinline__ T pair_diag(const PairRow<T> &P, const LevelK<T> &L, 
 // global load is issued before the first pass.  Any level of the plan
 // qualifies (odd sizes, semi-coarsening); the smoothing is the colour
 // passes of k_rb (pre: colour 0 first, post: colour 1 first).
-// From 16^3, FP32: 16.3 us a launch (27.5 with every operand in LDS, 64-bit
-// addresses formed again for each cell and a division an update; 5 us of it
-// is the loads).  FP64 from 16^3: 27 us, some registers spilled, against 12 us
-// from 8^3 and 27 us for the 16^3 level's own launches.
+// From 16^3, FP32: 15.5 us a launch (27.5 with every operand in LDS, 64-bit
+// addresses formed again for each cell and a division an update; 16.5 with
+// the inverse and the middle levels loaded after level 0 was formed).  FP64
+// from 16^3: 25.8 us, some registers spilled, against 12 us from 8^3 and 27 us
+// for the 16^3 level's own launches.
 // ---------------------------------------------------------------------
 constexpr int kTailMax = 8;
 constexpr int kTailThreads = 1024;
@@ -220,54 +229,88 @@ k_tail(TailK<T> K) {
     const LevelK<T> &L0 = K.L[0];
     const int np0 = (L0.nx + 1) >> 1, tot0 = np0 * L0.ny * L0.nz;
 
-    // level 0's rows and right-hand side
+    // Loads: level 0's couplings and right-hand side, those of a pair of the
+    // middle levels (all their pairs in turn, pair tid here) and four values
+    // of the inverse
     PairSet<T, DGI, P> S;
+    PairLoad<T, DGI> W[P], Wm;
+    T ba[P], bb[P], mv[4];
 #pragma unroll
     for (int p = 0; p < P; ++p) {
         const int e = tid + p * NT;
         S.on[p] = e < tot0;
         int m, j, k;
         split3(S.on[p] ? e : 0, np0, L0.ny, m, j, k);
-        load_pair<T, DGI>(L0, m, j, k, S.row[p]);
-        S.nb[p] = pair_nb(S.on[p] ? e : 0, m, j, k, np0, L0.ny, L0.nz);
+        W[p].load(L0, m, j, k);
         const int c = 2 * m + L0.nx * (j + L0.ny * k);
-        const bool two = 2 * m + 1 < L0.nx, odd = (j + k) & 1;
-        const T ba = K.b0[c], bb = two ? K.b0[c + 1] : (T)0;
-        S.b[p][0] = odd ? bb : ba;
-        S.b[p][1] = odd ? ba : bb;
+        ba[p] = K.b0[c];
+        bb[p] = K.b0[c + (2 * m + 1 < L0.nx ? 1 : 0)];
     }
-    // the inverse and the rows of the middle levels into LDS, the latter over
-    // all levels' pairs at once
-    for (int e = tid; e < nb * nb; e += NT) sm[K.off_minv + e] = K.minv[e];
-    {
-        int l = 1, base = 0;
-        for (int e = tid;; e += NT) {
-            int tot = 0;
-            for (; l < nl - 1; ++l) {
-                tot = pairs_of(K.L[l].nx, K.L[l].ny, K.L[l].nz);
-                if (e < base + tot) break;
-                base += tot;
-            }
-            if (l >= nl - 1) break;
-            const LevelK<T> &L = K.L[l];
-            const int p = e - base;
+    int at_m = 0, tm = 0, base = 0;   // Wm: its place in LDS, pairs of its level (0: none)
+    bool om = false, em = false;
+    for (int l = 1; l < nl - 1; ++l) {
+        const LevelK<T> &L = K.L[l];
+        const int tot = pairs_of(L.nx, L.ny, L.nz);
+        if (tid >= base && tid < base + tot) {
+            at_m = K.off_op[l] + tid - base;
+            tm = tot;
             int m, j, k;
-            split3(p, (L.nx + 1) >> 1, L.ny, m, j, k);
-            PairRow<T> row;
-            load_pair<T, DGI>(L, m, j, k, row);
-            T *o = sm + K.off_op[l] + p;
-            o[0] = row.co;
-#pragma unroll
-            for (int q = 0; q < 2; ++q) {
-                o[(1 + q) * tot] = row.cxo[q];
-                o[(3 + q) * tot] = row.cs[q];
-                o[(5 + q) * tot] = row.cn[q];
-                o[(7 + q) * tot] = row.cd[q];
-                o[(9 + q) * tot] = row.cu[q];
-                o[(11 + q) * tot] = row.rd[q];
-            }
+            split3(tid - base, (L.nx + 1) >> 1, L.ny, m, j, k);
+            om = 2 * m + 1 < L.nx;
+            em = (j + k) & 1;
+            Wm.load(L, m, j, k);
         }
+        base += tot;
     }
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+        if (tid + c * NT < nb * nb) mv[c] = K.minv[tid + c * NT];
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        const int e = S.on[p] ? tid + p * NT : 0;
+        int m, j, k;
+        split3(e, np0, L0.ny, m, j, k);
+        const bool two = 2 * m + 1 < L0.nx, odd = (j + k) & 1;
+        W[p].form(two, odd, S.row[p]);
+        S.nb[p] = pair_nb(e, m, j, k, np0, L0.ny, L0.nz);
+        if (!two) bb[p] = (T)0;
+        S.b[p][0] = odd ? bb[p] : ba[p];
+        S.b[p][1] = odd ? ba[p] : bb[p];
+    }
+    // the middle levels' rows and the inverse into LDS
+    auto rows_to_lds = [&](int at, int tot, const PairRow<T> &row) {
+        T *o = sm + at;
+        o[0] = row.co;
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            o[(1 + q) * tot] = row.cxo[q];
+            o[(3 + q) * tot] = row.cs[q];
+            o[(5 + q) * tot] = row.cn[q];
+            o[(7 + q) * tot] = row.cd[q];
+            o[(9 + q) * tot] = row.cu[q];
+            o[(11 + q) * tot] = row.rd[q];
+        }
+    };
+    if (tm) {
+        PairRow<T> row;
+        Wm.form(om, em, row);
+        rows_to_lds(at_m, tm, row);
+    }
+    for (int e = tid + NT; e < base; e += NT) {
+        int l = 1, p = e, tot;
+        for (; p >= (tot = pairs_of(K.L[l].nx, K.L[l].ny, K.L[l].nz)); ++l) p -= tot;
+        const LevelK<T> &L = K.L[l];
+        int m, j, k;
+        split3(p, (L.nx + 1) >> 1, L.ny, m, j, k);
+        PairRow<T> row;
+        Wm.load(L, m, j, k);
+        Wm.form(2 * m + 1 < L.nx, (j + k) & 1, row);
+        rows_to_lds(K.off_op[l] + p, tot, row);
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+        if (tid + c * NT < nb * nb) sm[K.off_minv + tid + c * NT] = mv[c];
+    for (int e = tid + 4 * NT; e < nb * nb; e += NT) sm[K.off_minv + e] = K.minv[e];
     auto rows_from_lds = [&](int l, int p, int tot, PairRow<T> &row) {
         const T *o = sm + K.off_op[l] + p;
         row.co = o[0];
