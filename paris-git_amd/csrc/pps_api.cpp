@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "pps_internal.h"
+#include "pps_stage.h"
 
 using namespace pps;
 
@@ -132,6 +133,9 @@ extern "C" int pps_finalize(pps_handle *h) {
     if (h->sorbox) (void)hipHostFree(h->sorbox);
     h->red.release();
     if (h->pinned) (void)hipHostFree(h->pinned);
+    if (h->stage.mem) (void)hipHostFree(h->stage.mem);
+    for (auto &e : h->stage.ev)
+        if (e) (void)hipEventDestroy(e);
     if (h->mbox) (void)hipHostFree(h->mbox);
     for (auto &e : h->prof.ev)
         if (e) (void)hipEventDestroy(e);
@@ -291,6 +295,11 @@ extern "C" int pps_set_cell_widths(pps_handle *h, const double *dx, const double
     return PPS_OK;
 }
 
+// a host array and its device copy
+static Span up_span(const DevBuf &d, const void *host, size_t n) {
+    return Span{(char *)d.ptr, (char *)const_cast<void *>(host), n};
+}
+
 // host-array staging shared by NewSolver / NewSolverMG
 static int host_solve(pps_handle *h, int method, const double *A, double *p, double maxError,
                       double beta, int maxit, int *it, int *ierr, int norm, double *tres2) {
@@ -302,14 +311,14 @@ static int host_solve(pps_handle *h, int method, const double *A, double *p, dou
     PPS_TRY(h->hA.ensure(bA));
     PPS_TRY(h->hp.ensure(bp));
     hipStream_t s = h->stream;
-    PPS_HIP(hipMemcpyAsync(h->hA.ptr, A, bA, hipMemcpyHostToDevice, s));
-    PPS_HIP(hipMemcpyAsync(h->hp.ptr, p, bp, hipMemcpyHostToDevice, s));
+    const Span in[2] = {up_span(h->hA, A, bA), up_span(h->hp, p, bp)};
+    PPS_TRY(stage_copy(h, in, 2, true, s));
     double t2 = 0.0;
     int rc = solve_with(h, method, h->hA.as<double>(), h->hp.as<double>(), maxError, beta, maxit,
                         norm, it, &t2, s);
     if (rc == PPS_OK || rc == PPS_ERR_NOT_CONVERGED) {
-        PPS_HIP(hipMemcpyAsync(p, h->hp.ptr, bp, hipMemcpyDeviceToHost, s));
-        PPS_HIP(hipStreamSynchronize(s));
+        const Span out{h->hp.as<char>(), (char *)p, bp};
+        PPS_TRY(stage_copy(h, &out, 1, false, s));
     }
     if (tres2) *tres2 = t2;
     // the reference reports the last MPI code in ierr; a failure aborts it
@@ -373,21 +382,17 @@ extern "C" int pps_free_solver(pps_handle *h, const double *A, double *p, const 
     PPS_TRY(h->hp.ensure(bp));
     PPS_TRY(h->hmask.ensure(bm));
     hipStream_t s = h->stream;
-    PPS_HIP(hipMemcpyAsync(h->hA.ptr, A, bA, hipMemcpyHostToDevice, s));
-    PPS_HIP(hipMemcpyAsync(h->hp.ptr, p, bp, hipMemcpyHostToDevice, s));
-    PPS_HIP(hipMemcpyAsync(h->hmask.ptr, pcmask, bm, hipMemcpyHostToDevice, s));
-    const double *dpg = nullptr;
-    if (P_gas) {
-        PPS_TRY(h->hpgas.ensure(bp));
-        PPS_HIP(hipMemcpyAsync(h->hpgas.ptr, P_gas, bp, hipMemcpyHostToDevice, s));
-        dpg = h->hpgas.as<double>();
-    }
+    if (P_gas) PPS_TRY(h->hpgas.ensure(bp));
+    const Span in[4] = {up_span(h->hA, A, bA), up_span(h->hp, p, bp), up_span(h->hmask, pcmask, bm),
+                        up_span(h->hpgas, P_gas, bp)};
+    PPS_TRY(stage_copy(h, in, P_gas ? 4 : 3, true, s));
+    const double *dpg = P_gas ? h->hpgas.as<double>() : nullptr;
     double t2 = 0.0;
     const int rc = free_with(h, h->hA.as<double>(), h->hp.as<double>(), h->hmask.as<int>(), dpg,
                              solver_flag, maxError, beta, maxit, it, &t2, s);
     if (rc == PPS_OK || rc == PPS_ERR_NOT_CONVERGED) {
-        PPS_HIP(hipMemcpyAsync(p, h->hp.ptr, bp, hipMemcpyDeviceToHost, s));
-        PPS_HIP(hipStreamSynchronize(s));
+        const Span out{h->hp.as<char>(), (char *)p, bp};
+        PPS_TRY(stage_copy(h, &out, 1, false, s));
     }
     if (tres2) *tres2 = t2;
     if (ierr) *ierr = (rc == PPS_OK || rc == PPS_ERR_NOT_CONVERGED) ? 0 : rc;
@@ -432,13 +437,13 @@ extern "C" int pps_poi_solve(pps_handle *h, const double *A, double *p, double m
     PPS_TRY(h->hA.ensure(bA));
     PPS_TRY(h->hp.ensure(bp));
     hipStream_t s = h->stream;
-    PPS_HIP(hipMemcpyAsync(h->hA.ptr, A, bA, hipMemcpyHostToDevice, s));
-    PPS_HIP(hipMemcpyAsync(h->hp.ptr, p, bp, hipMemcpyHostToDevice, s));
+    const Span in[2] = {up_span(h->hA, A, bA), up_span(h->hp, p, bp)};
+    PPS_TRY(stage_copy(h, in, 2, true, s));
     const int rc = poi_with(h, h->hA.as<double>(), h->hp.as<double>(), maxError, maxit, num_iterations,
                             solver_type, s);
     if (rc == PPS_OK || rc == PPS_ERR_NOT_CONVERGED) {
-        PPS_HIP(hipMemcpyAsync(p, h->hp.ptr, bp, hipMemcpyDeviceToHost, s));
-        PPS_HIP(hipStreamSynchronize(s));
+        const Span out{h->hp.as<char>(), (char *)p, bp};
+        PPS_TRY(stage_copy(h, &out, 1, false, s));
     }
     return rc;
 }

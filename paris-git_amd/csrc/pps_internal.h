@@ -154,6 +154,12 @@ struct SorBox {
 };
 constexpr int kSorBoxes = 8;
 
+// Pinned pieces (stage_copy) and the events that tell when each is free.
+struct StageRing {
+    char *mem = nullptr;
+    hipEvent_t ev[8] = {};
+};
+
 }  // namespace pps
 
 struct pps_handle {
@@ -186,6 +192,7 @@ struct pps_handle {
     double wmin = 1.0;
     pps::DevBuf red;               // reduction partials + results
     double *pinned = nullptr;      // 16 pinned host doubles for scalar readback
+    pps::StageRing stage;          // copies of a caller's pageable arrays (first large one)
     pps::Mailbox *mbox = nullptr;  // coherent host memory (pps_init)
     unsigned long long mseq = 0;   // seq of the last mailbox write requested
     pps::Prof prof;                // fine-level smoother timing
