@@ -1682,7 +1682,7 @@ k_update(long long n, double *__restrict__ r, const double *__restrict__ q, TB *
          double *__restrict__ S, double *__restrict__ part, AlphaK ak) {
     double alpha;
     if (ak.nb) {   // uniform
-        const double dq = sum_partials(part + 3 * kRedBlocks, ak.nb);
+        const double dq = sum_partials<4>(part + 3 * kRedBlocks, ak.nb);
         alpha = uniform(S[ak.rz] / dq);
         if (blockIdx.x == 0 && threadIdx.x == 0) {
             S[S_DQ] = dq;
@@ -2930,11 +2930,10 @@ static void queue_first(Hier<T> &H, const T *fineb, const Cycle &cy, hipStream_t
     else if (march_ok(H.lv[0], cy)) march_pre(H.lv[0], H.lv[1], fineb, cy, s, stop);
     else rb_sweep<T>(H.lv[0], 0, fineb, 0, true, cy, nullptr, s, nullptr, nullptr, stop.skip);
 }
-// Most partials of r.r that the queued kernel sums itself (the one-region
-// legs only).
+// Most partials of r.r that the queued kernel sums itself (the legs only).
 template <class T>
 static int fold_rr(const Hier<T> &H, const Cycle &cy) {
-    return leg_ok(H.lv[0], cy) ? kFoldParts : 0;
+    return leg_ok(H.lv[0], cy) || march_ok(H.lv[0], cy) ? kFoldWide : 0;
 }
 // Whether the look-ahead applies: the finest level runs legs or fused sweeps
 // and the cycle has a level below it.
@@ -3443,7 +3442,7 @@ static int outer_iterate(pps_handle *h, Hier<T> &H, bool mixed, double tol_abs, 
                                 : (fold ? k_dq_tiled<T, false, true> : k_dq_tiled<T, false, false>);
             kdq<<<tg.blocks, dim3(64, 16, 1), 0, s>>>(O, tg, z, dold, dnew, V.q, xu, S, part, bk);
             if (!lazy) p0 = k;   // d_(k-1) applied in k_dq_tiled
-            if (tg.blocks > kFoldParts) {
+            if (tg.blocks > kFoldWide) {
                 k_scal_alpha<<<1, 1024, 0, s>>>(part, ak, S);
                 ak.nb = 0;
             }

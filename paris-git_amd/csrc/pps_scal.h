@@ -21,12 +21,14 @@ static_assert(S_AH + kRingSlots <= 64, "ring alphas fit the scalars");
 
 // fixed-order sum of nb partials, the same value in every thread (any
 // block of at most 1024 threads whose x extent is a multiple of 64)
+template <int LOADS = 1>   // of a thread in flight
 __device__ __forceinline__ double sum_partials(const double *part, int nb) {
     __shared__ double sm[16];
     const int nt = blockDim.x * blockDim.y * blockDim.z;
     const int tid = threadIdx.x + blockDim.x * (threadIdx.y + blockDim.y * threadIdx.z);
     const int nw = nt >> 6;
     double v = 0.0;
+#pragma unroll LOADS
     for (int b = tid; b < nb; b += nt) v += part[b];
     v = wsum(v);
     if ((tid & 63) == 0) sm[tid >> 6] = v;
@@ -70,12 +72,18 @@ __device__ __forceinline__ double uniform(double v) {
     return u.d;
 }
 
-// Most partials that a consuming kernel's blocks sum themselves: the 32^3
-// solve (64 to 128 partials) saves its beta, alpha and r.r launches, 604 ->
-// 572 us.  At 64^3 (144 to 1024 partials) the kernels that take them over
-// grow by what the launches cost (908 against 919 us), and at 128^3 they lose
-// (1613 against 1632).
+// Most partials that a consuming kernel's blocks sum themselves.  Of beta's
+// (three sums, in k_dq_tiled): the 32^3 solve has 64 and saves the launch; at
+// 64^3 FP64 (144) k_dq_tiled would grow from 7.4 to 12.5 us, as much as the
+// kernel (4.1 us) and its gap take, and from 700 blocks on, two rounds on the
+// card, it would pay twice.
 constexpr int kFoldParts = 128;
+// Of alpha's (k_update) and r.r's (the next cycle's first leg), one sum: up to
+// 1024, a load for each thread of a leg and four for one of k_update.  128^3:
+// k_update 12.9 -> 13.3 us without k_scal_alpha's 4.2, k_march PRE 23.3 ->
+// 23.5 without k_scal_rr's 4.6; solves at 128^3 1576 -> 1555 us, 64^3 FP64 873
+// -> 860, 49x64x40 FP64 1088 -> 1060.
+constexpr int kFoldWide = 1024;
 
 // beta from the nb partials of (r, z), sum z, sum r: zmean, rho = r.(z - zmean),
 // beta = rho / rho_old, 0 in the first iteration.  rd, wr: the places of
