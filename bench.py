@@ -58,7 +58,7 @@ def level_dims(n3, periodic=(0, 0, 0), lengths=(1.0, 1.0, 1.0)):
     return dims
 
 
-def solve_bytes(n3, iters, S, nu_pre=2, nu_post=2, tail_cells=4096):
+def solve_bytes(n3, iters, S, tail_cells=4096):
     """Algorithmic bytes of one fast solve of a singular system whose A7 is
     the coupling sum (every array element counted once per launch that must
     touch it; S = bytes of the V-cycle type)."""
@@ -70,22 +70,24 @@ def solve_bytes(n3, iters, S, nu_pre=2, nu_post=2, tail_cells=4096):
         if li > 0 and n <= tail_cells:
             v += sum(x * y * z for (x, y, z) in dims[li:]) * S * 5    # LDS tail: staged once
             break
-        v += n * S * (5 + 6 * (nu_pre - 1))                 # pre-smoothing (first: no x read)
-        v += n * S * ((6 + 1 / 8) + 6 * (nu_post - 1))      # post (first adds the correction)
-        v += n * S * (5 + 1 / 8)                            # residual + restriction
+        # a leg is one pass: couplings and b in, the first colour of x and
+        # the coarse b out; those, half of x and the correction in, x out
+        v += n * S * (4.5 + 1 / 8)
+        v += n * S * (5.5 + 1 / 8)
     else:
         nb = dims[-1][0] * dims[-1][1] * dims[-1][2]
         v += nb * nb * S + 2 * nb * S                       # dense bottom solve
     mixed = S == 4
-    # the PCG step: (r, z) comes with the last sweep; d & A d reads z, d_old,
-    # the FP64 couplings and x (the previous x += alpha d), writes d (type
-    # S), q and x; the update reads r, q and writes r (+ its FP32 copy)
-    outer = n0 * ((48 + 3 * S) + (24 + (4 if mixed else 0)))
+    # the PCG step: (r, z) comes with the last leg; d & A d reads z, d_old and
+    # the FP64 couplings, writes d (type S) and q; the update reads r, q and
+    # writes r (+ its FP32 copy); x += alpha d of all but the last direction
+    # in one pass at the end
+    outer = n0 * ((32 + 3 * S) + (24 + (4 if mixed else 0)))
     setup = n0 * (72 + 56 + (20 if mixed else 0))           # A, p in; op, b, x, r (+ FP32) out
     for (a, b, c) in dims[1:]:
         setup += a * b * c * S * (8 * 4 + 4)                # coarsening
-    final = n0 * (16 + S)                                   # the last x += alpha d
-    final += n0 * (40 + 8)                                  # true residual + write-back of p
+    final = n0 * (16 + (iters - 1) * S)                     # the deferred x += alpha d
+    final += n0 * (48 + S)                                  # the last one, true residual, p
     return setup + iters * (v + outer) + final
 
 
@@ -93,7 +95,7 @@ TRAFFIC_FILE = os.path.join(ROOT, "profiles", "k_march_drops256_traffic.md")
 
 
 def measured_traffic():
-    """HBM bytes per launch of the profiled sweep kernel, from the committed
+    """HBM bytes per launch of the profiled smoothing kernel, from the committed
     counter summary (FETCH_SIZE + WRITE_SIZE, calibrated against a copy of
     known size); None when no summary is present."""
     try:
@@ -112,7 +114,7 @@ def gpu_run(pps, torch, grid, A, method, tol, steps, warmup, maxit=200):
     for _ in range(warmup):
         p.zero_()
         s.solve(A, p, tol, 1.2, maxit, allow_maxit=False)
-    # one launch in 7 of the timed sweep kernel carries the event pair (7 is
+    # one launch in 7 of the timed smoothing kernel carries the event pair (7 is
     # prime to the iteration count, so the samples rotate through the cycles)
     s.profile(True, every=7)
     s.profile_read()
