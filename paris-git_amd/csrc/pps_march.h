@@ -41,11 +41,13 @@
 // value a pair.  After PRE's last pass the residual of colour 1 is zero (its
 // equations were just solved), so only colour 0's is formed.
 //
-// A cell outside a wall, a missing second cell of an odd row and the edge of
-// the region carry finite junk (the nearest cell's row): a cell inside has
-// coupling 0 to them, or no output depends on them.  Planes beyond a wall are
-// zero.  A periodic axis wraps.  Singular systems only (every diagonal is
-// the coupling sum).
+// What lies beyond a wall (cells, planes) and the missing second cell of an
+// odd row are inert: no couplings, reciprocal diagonal 0, value 0.  Cells
+// inside reach them through couplings of 0 only, but zero times a value is
+// zero only if that is finite, and the row of the nearest cell in their place
+// can have a diagonal of 0 (its one open face the one towards the cells
+// inside).  No output depends on the edge of the region.  A periodic axis
+// wraps.  Singular systems only (every diagonal is the coupling sum).
 #pragma once
 
 #include "pps_leg.h"
@@ -170,6 +172,8 @@ k_march(LevelK<T> L, MarchK g, Coarsening cg, const T *__restrict__ b, const T *
     const int ui = ox - kMarchHalo + 2 * m, uj = oy - kMarchHalo + j;
     const int gi = place(ui, nx, g.px) & ~1, gj = place(uj, ny, g.py);
     const bool two = V16 || gi + 1 < nx;     // the pair's second cell exists
+    // the pair's first cell lies in the level
+    const bool real = (g.px || (ui >= 0 && ui < nx)) && (g.py || (uj >= 0 && uj < ny));
     const bool mine = m >= 2 && m < kR - 2 && j >= 4 && j < 28 && ui < nx && uj < ny;
     const bool wallw = ui == 0 && !g.px, walls = uj == 0 && !g.py;   // no coupling to the left, below
     const long long sz = (long long)nx * ny, n = sz * nz;
@@ -330,7 +334,7 @@ k_march(LevelK<T> L, MarchK g, Coarsening cg, const T *__restrict__ b, const T *
         if (!LATE) ahead = request(An, s + 2, E);
         if (PRE && s - 5 >= k0) finish(s - 5, 1 - E);
         // plane s
-        if (plane_of(s) >= 0) {
+        if (plane_of(s) >= 0 && real) {
             const LdsPair<T> vx = A.cx[own], vn = A.cy[own], vs = A.cy[rs], vu = A.cz[own], vb = A.b[own];
             T left = beside<false, kR>(vx.b);
             if (PRE) left = m == 0 ? A.e0[jh + 16 * jl] : left;
@@ -343,8 +347,8 @@ k_march(LevelK<T> L, MarchK g, Coarsening cg, const T *__restrict__ b, const T *
             cu[P0][0] = vu.a; cu[P0][1] = vu.b;
             bb[P0][0] = vb.a; bb[P0][1] = vb.b;
             rd[P0][0] = (T)1 / diag_sum(cx[P0][0], co[P0], cs[P0][0], cn[P0][0], cu[P1][0], cu[P0][0]);
-            rd[P0][1] = (T)1 / diag_sum(co[P0], cx[P0][1], cs[P0][1], cn[P0][1], cu[P1][1], cu[P0][1]);
-            xr[P0] = PRE ? bb[P0][E] * rd[P0][E] : A.e0[own] + A.e1[own];
+            rd[P0][1] = two ? (T)1 / diag_sum(co[P0], cx[P0][1], cs[P0][1], cn[P0][1], cu[P1][1], cu[P0][1]) : (T)0;
+            xr[P0] = PRE ? bb[P0][E] * rd[P0][E] : E == 1 && !two ? (T)0 : A.e0[own] + A.e1[own];
         } else {
             co[P0] = xr[P0] = (T)0;
 #pragma unroll

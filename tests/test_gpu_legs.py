@@ -116,3 +116,45 @@ def test_repeated_solves_swap_buffers(pps):
             it, _ = s.solve(A, p, 1e-10 * brms, 1.2, 60, allow_maxit=False)
             print(f"after {its} cycles: {it} iterations", flush=True)
             assert it <= 15
+
+
+@pytest.mark.parametrize("closed", [0.0, 1e-44])
+@pytest.mark.parametrize("method", ["fp64", "mixed"])
+@pytest.mark.parametrize("shape,bc", [
+    ((72, 72, 72), WALLS),    # 16-byte loads in both precisions
+    ((66, 70, 76), WALLS),    # 16-byte loads in FP64, 4-byte ones in FP32
+    ((73, 67, 71), WALLS),    # 4-byte loads, missing second cells
+    ((64, 81, 70), PX),       # walls in y and z only
+])
+def test_marching_legs_with_cells_open_to_one_side(pps, shape, bc, method, closed):
+    """Dead ends of one cell (faces closed by the masks, or all but closed: their
+    couplings are FP32 denormals) at the walls and beside them.  A marching leg
+    holds cells beyond a wall; whatever it takes as their rows, they must not
+    reach the cells inside through couplings of zero."""
+    print("dead ends", shape, bc, method, closed, flush=True)
+    g = pps.Grid.make(*shape, bdry_cond=bc)
+    rho, u, v, w = pps.synth_fields(g, [(0.4, 0.5, 0.5, 0.2), (0.8, 0.3, 0.6, 0.12)], 1.0, 100.0, 1.5, seed=4)
+    masks = pps.pressure_masks(g)
+    nx, ny, nz = shape
+    ends = [((11, ny - 1, 9), (1, -1)), ((30, 0, 21), (1, 1)), ((37, 40, nz - 1), (2, -1)), ((20, 33, 0), (2, 1))]
+    if not bc[0]:   # at the x walls; those of 16 bytes before the high one
+        ends += [((nx - q, 9 + 8 * q, 13 + 6 * q), (0, -1)) for q in (1, 2, 3, 4)]
+        ends += [((0, 25, 31), (0, 1)), ((nx - 1, ny - 1, 44), (1, -1)), ((nx - 1, ny - 1, 50), (0, -1))]
+    for cell, way in ends:
+        for a in range(3):
+            for side in (-1, 1):
+                c = list(cell)
+                c[a] += min(side, 0)
+                if (a, side) != way and 0 <= c[a] < shape[a] - 1:   # a wall's faces are closed
+                    masks[a][g.ng + c[2], g.ng + c[1], g.ng + c[0]] = closed
+    A = pps.setup_poisson(g, u, v, w, *masks, rho, 1.0)
+    pps.remove_rhs_mean(g, A)
+    for cell, way in ends:
+        open_ = A[:6, cell[2], cell[1], cell[0]] > 1e-30
+        assert open_.nonzero().flatten().tolist() == [2 * way[0] + (way[1] > 0)]
+    x = _cycle(pps, g, A, method)
+    ref = _cycle(pps, g, A, method, smoother=pps.SMOOTH_COLOUR_PASSES, tail_cells=-1)
+    assert bool(torch.isfinite(ref).all())
+    err = float((x - ref).abs().max() / ref.abs().max())
+    print(f"   err {err:.2e}", flush=True)
+    assert err <= TOL[method]
