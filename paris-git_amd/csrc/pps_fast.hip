@@ -1888,7 +1888,8 @@ k_unpack(PackK d, const double *__restrict__ x, double *__restrict__ p) {
 // residual r = A8 - A7 p + sum A_nb p_nb (the reference's own expression
 // on the padded p, MGsolver.f90:97-100), and in mixed mode the FP32 copies
 // of the operator and of r.  Partials: 0 = sum r^2, 1 = sum b^2.  flags as
-// k_pack, plus bit3: some A7 differs from the coupling sum outer_diag forms.
+// k_pack, plus bit3: some A7 differs from the coupling sum outer_diag forms;
+// bit4 (mixed mode): a coupling other than 0, or a diagonal, is below tiny.
 // W (wx, wy, wz not null): every row is first multiplied by the weight
 // w = wx[i] wy[j] wz[k] (normalised cell volumes), which makes the system
 // of a stretched grid symmetric: SetupPoisson's couplings of a face are
@@ -2015,7 +2016,7 @@ k_setup(PackK d, int zc, Src src, const double *__restrict__ p,
         double *__restrict__ dg, double *__restrict__ bo, double *__restrict__ x,
         double *__restrict__ r, float *__restrict__ f32, float *__restrict__ r32,
         double *__restrict__ part, int *__restrict__ flags, const double *__restrict__ wx,
-        const double *__restrict__ wy, const double *__restrict__ wz) {
+        const double *__restrict__ wy, const double *__restrict__ wz, double tiny) {
     const int i = blockIdx.x * 64 + threadIdx.x;
     const int j = blockIdx.y * 4 + threadIdx.y;
     const int k0 = blockIdx.z * zc;
@@ -2105,6 +2106,10 @@ k_setup(PackK d, int zc, Src src, const double *__restrict__ p,
                 f32[c] = (float)vx; f32[n + c] = (float)vy; f32[2 * n + c] = (float)vz;
                 if (Src::kDiagStored) f32[3 * n + c] = (float)a[6];
                 r32[c] = (float)rv;
+                // (all of a singular system's diagonals are at least its
+                // least coupling other than 0)
+                auto small = [&](double v) { return v != 0.0 && fabs(v) < tiny; };
+                if (small(vx) || small(vy) || small(vz) || a[6] < tiny) f |= 16;
             }
             rr += rv * rv;
             bb += wx ? (rhs / wc) * (rhs / wc) : rhs * rhs;
@@ -2320,6 +2325,7 @@ struct FastState {
     DevBuf flags;
     int singular = 1;
     int exact = 0;   // every A7 is the coupling sum of outer_diag, bit for bit
+    int tiny = 0;    // FP32 diagonals of the hierarchy may have no finite reciprocal
     const double *built_for = nullptr;
     const double *built_w[3] = {nullptr, nullptr, nullptr};   // face weights (face-value systems)
     int built_mixed = 0;   // precision of the hierarchy last built for built_for
@@ -2657,6 +2663,7 @@ struct Cycle {
     int nu_pre = 2, nu_post = 2;
     bool dgi = false, fused = true;
     bool tri = false;          // trilinear transfers
+    bool divide = false;       // diagonals without a reciprocal: the kernels that divide by them
     int per[3] = {0, 0, 0};    // periodic axes
     int rows = 0, planes = 0;
     long long tail_cells = 4096;
@@ -2814,7 +2821,7 @@ template <class T> constexpr long long kLegCells = sizeof(T) == 4 ? 300000 : 150
 template <class T>
 static bool leg_ok(const Level<T> &L, const Cycle &cy) {
     return cy.fused && !cy.tri && cy.nu_pre == 2 && cy.nu_post == 2 && cy.rows == 0 && cy.planes == 0 &&
-           L.n <= kLegCells<T>;
+           L.n <= kLegCells<T> && !cy.divide;
 }
 // Planes of a leg's region (its outputs take 8 fewer): 16, or in FP32, whose
 // registers hold three pairs a thread, 24 where that still gives every CU a
@@ -2873,7 +2880,7 @@ static int leg_post(Level<T> &L, int l, const Level<T> &C, const T *b, const Cyc
 // the one-region legs; 64^3 FP32 15 + 13 against their 9.1 + 9.3.
 template <class T>
 static bool march_ok(const Level<T> &L, const Cycle &cy) {
-    return cy.fused && !cy.tri && cy.dgi && cy.nu_pre == 2 && cy.nu_post == 2 && cy.rows == 0 && cy.planes == 0 &&
+    return cy.fused && !cy.tri && cy.dgi && !cy.divide && cy.nu_pre == 2 && cy.nu_post == 2 && cy.rows == 0 && cy.planes == 0 &&
            L.n > kLegCells<T> && L.n * (long long)sizeof(T) < (1LL << 32) && L.nx >= 16 && L.ny >= 16 && L.nz >= 8;
 }
 // Blocks of a marching leg: the planes of a block that minimise rounds of
@@ -2971,7 +2978,7 @@ static int vcycle(Hier<T> &H, const T *fineb, const Cycle &cy, Prof *prof, hipSt
             return lds > 0 && lds <= cy.lds_max;
         };
         while (lt < nl && !fits(lt)) ++lt;
-        if (lt == nl - 1) lt = nl;
+        if (lt == nl - 1 || (cy.divide && !cy.tri)) lt = nl;
     }
     // the coarse operators (built on the side stream) are needed once the
     // finest level's smoothing and restriction, which only write the coarse
@@ -3227,6 +3234,10 @@ static int fast_setup(pps_handle *h, const double *dA, const double *dp, bool mi
         f32 = f->h32.lv[0].cx;   // cx, cy, cz, dg are contiguous
         r32 = f->b32.as<float>();
     }
+    // The legs and the tail multiply by the reciprocals of the diagonals, which
+    // overflow for FP32 denormals: every level's diagonals must be normal.  A
+    // coarse coupling is 0 or at least 1/16 of the least fine one.
+    const double tiny = std::ldexp(1.0, -126 + 4 * ((int)dims.size() / 3 - 1));
     // operator, right-hand side, iterate and initial residual in one pass
     double *part = f->red.as<double>();
     double *S = part + 4 * kRedBlocks;
@@ -3244,15 +3255,15 @@ static int fast_setup(pps_handle *h, const double *dA, const double *dp, bool mi
     if (rows) {
         const RowsF src{*rows, d.nx, d.ny, d.nz, d.ng, (long long)d.X(), (long long)d.X() * d.Y()};
         k_setup<RowsF><<<zg.grid, dim3(64, 4, 1), 0, s>>>(packk(d), zg.zc, src, dp, ocx, ocy, ocz, odg, V.b,
-                                                          V.x, V.r, f32, r32, part, flags, wx, wy, wz);
+                                                          V.x, V.r, f32, r32, part, flags, wx, wy, wz, tiny);
     } else if (faces) {
         const RowsC src{*faces, d.nx, d.ny, d.nz, d.per[0], d.per[1], d.per[2], {0.0, 0.0, 0.0}};
         k_setup<RowsC><<<zg.grid, dim3(64, 4, 1), 0, s>>>(packk(d), zg.zc, src, dp, ocx, ocy, ocz, odg, V.b,
-                                                          V.x, V.r, f32, r32, part, flags, wx, wy, wz);
+                                                          V.x, V.r, f32, r32, part, flags, wx, wy, wz, tiny);
     } else {
         const RowsA src{dA, n, 0.0};
         k_setup<RowsA><<<zg.grid, dim3(64, 4, 1), 0, s>>>(packk(d), zg.zc, src, dp, ocx, ocy, ocz, odg, V.b,
-                                                          V.x, V.r, f32, r32, part, flags, wx, wy, wz);
+                                                          V.x, V.r, f32, r32, part, flags, wx, wy, wz, tiny);
     }
     // deferred: r.r, b.b and the flags go to the mailbox as well
     if (defer) k_scal_rr<<<1, 1024, 0, s>>>(part, zg.blocks, 1, S, 1, h->mbox, ++h->mseq, flags);
@@ -3291,6 +3302,7 @@ static int fast_setup(pps_handle *h, const double *dA, const double *dp, bool mi
         if (fl & 2) return PPS_ERR_NONSYMMETRIC;
         f->singular = (fl & 4) ? 0 : 1;
         f->exact = (fl & 8) ? 0 : 1;
+        f->tiny = (fl & 16) ? 1 : 0;
         PPS_TRY(build(f->singular, s));
     }
     f->have_r = 1;
@@ -3352,6 +3364,7 @@ static int outer_iterate(pps_handle *h, Hier<T> &H, bool mixed, double tol_abs, 
         }
         f->singular = (fl & 4) ? 0 : 1;
         f->exact = (fl & 8) ? 0 : 1;
+        f->tiny = (fl & 16) ? 1 : 0;
         if (!f->singular) {
             // built for a singular system on the side stream: build again
             // with the stored diagonals, after that build
@@ -3368,6 +3381,7 @@ static int outer_iterate(pps_handle *h, Hier<T> &H, bool mixed, double tol_abs, 
     cy.fused = h->opt.smoother != PPS_SMOOTH_COLOUR_PASSES;
     cy.rows = h->opt.sweep_rows;
     cy.planes = h->opt.sweep_planes;
+    cy.divide = sizeof(T) == 4 && f->tiny;
     cy.tail_cells = h->opt.tail_cells == 0 ? 4096 : (h->opt.tail_cells < 0 ? 0 : h->opt.tail_cells);
     cy.lds_max = f->lds_max;
     cy.cus = f->cus;

@@ -158,3 +158,34 @@ def test_marching_legs_with_cells_open_to_one_side(pps, shape, bc, method, close
     err = float((x - ref).abs().max() / ref.abs().max())
     print(f"   err {err:.2e}", flush=True)
     assert err <= TOL[method]
+
+
+@pytest.mark.parametrize("closed", [1e-40, 1e-44])
+@pytest.mark.parametrize("shape", [(48, 48, 48), (72, 72, 72), (73, 67, 71)])
+def test_mixed_solve_with_denormal_couplings(pps, shape, closed):
+    """A block whose faces are all but closed: in FP32 its diagonals are
+    denormals, whose reciprocals overflow.  The mixed solve must converge as the
+    FP64 one does (two iterations allowed for the precision)."""
+    print("denormal block", shape, closed, flush=True)
+    g = pps.Grid.make(*shape)
+    rho, u, v, w = pps.synth_fields(g, [(0.4, 0.5, 0.5, 0.2)], 1.0, 100.0, 1.5, seed=4)
+    masks = list(pps.pressure_masks(g))
+    block = torch.zeros(g.shape_p, dtype=torch.bool, device="cuda")
+    lo, hi = g.ng + shape[0] // 4, g.ng + shape[0] // 2
+    block[lo:hi, lo:hi, lo:hi] = True
+    for a in range(3):
+        faces = (block | torch.roll(block, -1, 2 - a)) & (masks[a] > 0)
+        masks[a][faces] = closed
+        (u, v, w)[a][faces] = 0.0
+    A = pps.setup_poisson(g, u, v, w, *masks, rho, 1.0)
+    inside = g.interior(block)
+    A[7][inside] = 0.0
+    A[7][~inside] -= A[7].sum() / (~inside).sum()
+    tol = 1e-10 * float((A[7] ** 2).mean().sqrt())
+    its = {}
+    for method in ("fp64", "mixed"):
+        with pps.Solver(g, method=method) as s:
+            p = torch.zeros(g.shape_p, dtype=torch.float64, device="cuda")
+            its[method] = s.solve(A, p, tol, 1.2, 60, allow_maxit=False)[0]
+    print("   iterations", its, flush=True)
+    assert its["mixed"] <= its["fp64"] + 2
