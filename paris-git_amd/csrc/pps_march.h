@@ -259,7 +259,10 @@ k_march(LevelK<T> L, MarchK g, Coarsening cg, const T *__restrict__ b, const T *
     // outstanding: its loads for plane s + 2 and both steps' stores, which
     // stay in flight (to wait for one of those loads costs a memory latency a
     // step: 256^3 FP32 PRE 99 us, POST 135; counted 95 and 124).  A count too
-    // low is safe.
+    // low is safe; one that takes in a store older than the loads waited for
+    // is not, so a wavefront that requests at the start of a step must issue
+    // those loads before the step's stores, which touch other memory: the
+    // empty asm there keeps the order.
     constexpr int kLoads = (V16 ? 1 : 4) * NC + (PRE ? 0 : 2 * DW);
 
     // rows of the last planes by position, and the values of both colours in
@@ -331,7 +334,10 @@ k_march(LevelK<T> L, MarchK g, Coarsening cg, const T *__restrict__ b, const T *
             return v;
         };
         bool ahead = false;
-        if (!LATE) ahead = request(An, s + 2, E);
+        if (!LATE) {
+            ahead = request(An, s + 2, E);
+            asm volatile("" ::: "memory");   // before this step's stores (see kLoads)
+        }
         if (PRE && s - 5 >= k0) finish(s - 5, 1 - E);
         // plane s
         if (plane_of(s) >= 0 && real) {
