@@ -548,7 +548,7 @@ int ref_solve(pps_handle *h, const double *dA, double *dp, double maxError,
     return PPS_OK;
 }
 
-// RB-SOR iterations on the colour-split A for at most maxit iterations: on
+// RB-SOR iterations on the colour-split A for at most maxit (1 or more): on
 // the stream, iteration k's first pass (which also forms the statistics of
 // iteration k-1's first colour), the totals of iteration k-1, iteration k's
 // second pass.  The host queues kSorAhead iterations beyond the one whose
@@ -756,7 +756,8 @@ int free_solve(pps_handle *h, const double *dA, double *dp, const int *dmask, co
     PPS_TRY(rc);
     dim3 sgrid, tgrid;
     int nbk = 0, k;
-    if (As && sor_shapes(L, &sgrid, &tgrid, &nbk)) {
+    // (a limit below 1 runs none: the loop below)
+    if (As && maxit > 0 && sor_shapes(L, &sgrid, &tgrid, &nbk)) {
         double sum = 0.0;
         int stopped;
         bool bad;

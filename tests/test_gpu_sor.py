@@ -68,3 +68,30 @@ def test_new_solver_std_diverges_where_the_oracle_does(pps, orc, shape, bc):
         assert e.value.code == pps.ERR_DIVERGED
         assert len(s.history()) == it - 1
     _same(og, p, want, 1e-9)
+
+
+def test_free_solver_without_iterations(pps, orc):
+    """A limit below 1 runs none: it = 1 (a loop of no trips, as the oracle's),
+    and the handle's later calls see their own totals."""
+    g, og, At, A = _system(pps, orc, (32, 24, 20), WALLS)
+    m = torch.zeros(g.shape_p, dtype=torch.int32, device="cuda")
+    m[10, 12, 14] = 1
+    pgas = torch.ones(g.shape_p, dtype=torch.float64, device="cuda")
+
+    def call(s, limit):
+        p = torch.zeros(g.shape_p, dtype=torch.float64, device="cuda")
+        it, t2 = s.free_solve(At, p, m, pgas, 1, 0.0, 1.2, limit)
+        return it, t2, list(s.history()), p
+
+    with pps.Solver(g, method="sor") as s:
+        first = call(s, 5)
+        assert first[0] == 6 and len(first[2]) == 5
+        for limit in (0, -1, -3):
+            print("free solver limit", limit, flush=True)
+            want = np.zeros(og.shape_p)
+            rc, it, t2, _ = orc.free_solver(og, A, want, m.cpu().numpy(), pgas.cpu().numpy(), 1, 0.0, 1.2, limit)
+            none = call(s, limit)
+            assert rc == 0 and none[:3] == (it, t2, [])
+            assert np.array_equal(og.interior(none[3].cpu().numpy()), og.interior(want))
+            again = call(s, 5)
+            assert again[:3] == first[:3] and torch.equal(again[3], first[3])
