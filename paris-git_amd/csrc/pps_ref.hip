@@ -115,21 +115,28 @@ __device__ __forceinline__ double blk_red(double v, double *sm, bool mx, int t) 
 // values that the update reads anyway (PASS_FIRST; it keeps what it
 // overwrites in old, one value a pair, for an iteration that turns out to be
 // the last one); after the last iteration, in a pass of their own
-// (PASS_STATS).  128^3: 53 us an iteration's passes against 73 with a
-// statistics pass of its own in every one (67 MB of A each).
+// (PASS_STATS).  The first iteration's first pass has none to form
+// (PASS_START; it clears *stop).  128^3: 53 us an iteration's passes against
+// 73 with a statistics pass of its own in every one (67 MB of A each).
 // The statistics equal k_resid_stats_fs's (same residual expression, sums
 // in another order).  Block partials {sum r^2, max |r|, active cells, NaN
 // cells} at part[c * kRedBlocks + boff + block].  !FS: every cell, the
 // residual of MGsolver.f90:97-100 as compute_residual_norm forms it, partial
 // 0 = sum |r|^norm.  Nothing is done once *stop is set.
-enum { PASS_FIRST, PASS_SECOND, PASS_STATS };
+enum { PASS_START, PASS_FIRST, PASS_SECOND, PASS_STATS };
 template <int PASS, bool FS>
 __global__ void __launch_bounds__(256)
 k_sor_pass(LvlK L, const double *__restrict__ As, double *__restrict__ p,
                 const int *__restrict__ pcmask, int flag, double beta, int colour,
                 double *__restrict__ part, int boff, int norm, double *__restrict__ old,
-                const int *__restrict__ stop) {
-    if (*stop) return;
+                int *__restrict__ stop) {
+    const int t = threadIdx.x + 64 * threadIdx.y;
+    const long long blk = blockIdx.x + (long long)gridDim.x * (blockIdx.y + (long long)gridDim.y * blockIdx.z);
+    if (PASS == PASS_START) {
+        if (blk == 0 && t == 0) *stop = 0;
+    } else if (*stop) {
+        return;
+    }
     __shared__ double sm[4];
     const long long hn = lk_cells(L) / 2;
     const int hx = L.nx / 2;
@@ -155,6 +162,7 @@ k_sor_pass(LvlK L, const double *__restrict__ As, double *__restrict__ p,
             pnew = (1.0 - beta) * pc + beta / a[6 * hn + h] * s;
             p[q] = pnew;
         }
+        if (PASS == PASS_START) continue;
         if (PASS == PASS_FIRST) old[h] = pc;
         if (PASS == PASS_SECOND) pc = pnew;
         if (!FS) {
@@ -174,8 +182,8 @@ k_sor_pass(LvlK L, const double *__restrict__ As, double *__restrict__ p,
         cnt += 1.0;
         if (nan) bad += 1.0;
     }
-    const int t = threadIdx.x + 64 * threadIdx.y;
-    const long long b = boff + blockIdx.x + (long long)gridDim.x * (blockIdx.y + (long long)gridDim.y * blockIdx.z);
+    if (PASS == PASS_START) return;
+    const long long b = boff + blk;
     double v = blk_red(s2, sm, false, t);
     if (t == 0) part[b] = v;
     if (!FS) return;
@@ -244,10 +252,6 @@ k_sor_undo(LvlK L, double *__restrict__ p, const int *__restrict__ pcmask, int f
     const long long q = ipad(L, 2 * m + ((j + k) & 1), j, k);
     if (FS && !(flag == 1 ? pcmask[q] == 0 : (pcmask[q] == 1 || pcmask[q] == 2))) return;
     p[q] = old[((long long)k * L.ny + j) * (L.nx / 2) + m];
-}
-
-__global__ void __launch_bounds__(64) k_sor_start(int *stop) {
-    if (threadIdx.x == 0) *stop = 0;
 }
 
 // One-layer periodic wrap of the face ghosts of a level.
@@ -551,12 +555,17 @@ int ref_solve(pps_handle *h, const double *dA, double *dp, double maxError,
 // RB-SOR iterations on the colour-split A for at most maxit (1 or more): on
 // the stream, iteration k's first pass (which also forms the statistics of
 // iteration k-1's first colour), the totals of iteration k-1, iteration k's
-// second pass.  The host queues kSorAhead iterations beyond the one whose
-// totals it waits for, so the device does not idle while they travel: once
-// the totals set the stop flag the passes behind them return at once, and
-// the one first pass that ran before them is undone.  Gives the iteration
-// that stopped (0: none did) and the totals of the last one; each
-// iteration's totals are passed to `seen`.
+// second pass.  The host queues up to kSorAhead iterations beyond the one
+// whose totals it waits for, so the device does not idle while they travel:
+// once the totals set the stop flag the passes behind them return at once, and
+// the one first pass that ran before them is undone.  It looks for the totals
+// before each launch: a call of few iterations is mostly launches (a limit of
+// 2 at 32^3 70 us, 79 with all queued first).  A call that stops in its first
+// iteration pays for the pass undone: 32^3 74 us, 256^3 1042, against 64 and
+// 968 with a statistics pass in every iteration; from the second on it gains
+// (32^3 84 against 86, 256^3 1412 against 1487).
+// Gives the iteration that stopped (0: none did) and the totals of the last
+// one; each iteration's totals are passed to `seen`.
 constexpr int kSorAhead = 2;
 static_assert(kSorAhead + 2 <= kSorBoxes, "a slot for every iteration in flight");
 template <bool FS, class Seen>
@@ -573,18 +582,20 @@ static int sor_split(pps_handle *h, const LvlK &L, const double *As, double *dp,
         PPS_HIP(hipHostMalloc((void **)&h->sorbox, kSorBoxes * sizeof(SorBox), hipHostMallocCoherent));
         for (int q = 0; q < kSorBoxes; ++q) h->sorbox[q].seq = 0;
     }
-    k_sor_start<<<1, 64, 0, s>>>(stop);
     const unsigned long long base = h->sorseq;
     h->sorseq += (unsigned long long)maxit;
     auto box = [&](int k) { return h->sorbox + (base + k) % kSorBoxes; };
     auto totals = [&](int k) {
         k_sor_final<FS><<<1, 1024, 0, s>>>(part, 2 * nbk, N, norm, maxError, box(k), base + k, stop);
     };
-    auto queue = [&](int k) {
-        k_sor_pass<PASS_FIRST, FS><<<tgrid, kCellBlock, 0, s>>>(L, As, dp, dmask, flag, beta, 0, part, nbk, norm,
-                                                               old, stop);
+    auto arrived = [&](int k) { return __atomic_load_n(&box(k)->seq, __ATOMIC_ACQUIRE) == base + k; };
+    auto first = [&](int k) {
+        auto pass = k > 1 ? k_sor_pass<PASS_FIRST, FS> : k_sor_pass<PASS_START, FS>;
+        pass<<<tgrid, kCellBlock, 0, s>>>(L, As, dp, dmask, flag, beta, 0, part, nbk, norm, old, stop);
         launch_halo(L, dp, s);
         if (k > 1) totals(k - 1);
+    };
+    auto second = [&](int k) {
         k_sor_pass<PASS_SECOND, FS><<<tgrid, kCellBlock, 0, s>>>(L, As, dp, dmask, flag, beta, 1, part, 0, norm,
                                                                 old, stop);
         launch_halo(L, dp, s);
@@ -596,16 +607,19 @@ static int sor_split(pps_handle *h, const LvlK &L, const double *As, double *dp,
     };
     *stopped = 0;
     *bad = false;
-    int queued = 0;
+    int q1 = 0, q2 = 0;   // first and second passes queued
     for (int k = 1; k <= maxit; ++k) {
         // iteration k's totals come with iteration k+1's first pass
-        while (queued < maxit && queued < k + kSorAhead) queue(++queued);
+        while (q2 < maxit && q2 < k + kSorAhead && !arrived(k)) {
+            if (q1 == q2) first(++q1);
+            else second(++q2);
+        }
         PPS_HIP(hipGetLastError());
         const SorBox *b = box(k);
-        for (long long spin = 1; __atomic_load_n(&b->seq, __ATOMIC_ACQUIRE) != base + k; ++spin) {
+        for (long long spin = 1; !arrived(k); ++spin) {
             if ((spin & 255) == 0) {
                 const hipError_t e = hipStreamQuery(s);
-                if (e == hipSuccess && __atomic_load_n(&b->seq, __ATOMIC_ACQUIRE) != base + k) {
+                if (e == hipSuccess && !arrived(k)) {
                     std::fprintf(stderr, "libpps: the stream drained without the expected reduction\n");
                     return PPS_ERR_HIP;
                 }
