@@ -2814,9 +2814,14 @@ static void rb_sweep(Level<T> &L, int l, const T *b, int c1, bool first, const C
 // Whether level l's smoothing legs run as one launch each (k_leg_pre,
 // k_leg_post): the default cycle, on levels small enough that the sweeps'
 // launches cost more than the cells that the legs compute several times
-// over.  FP32: 64^3 9.1 + 9.3 us against 17.4 + 14.6 for the sweeps, 100^3
-// 34 + 51 against 32 + 27.  FP64: 32^3 8.3 + 7.5 us against 16.5 + 10.6, 64^3
-// 17.5 + 19.8 against 29 + 19.
+// over.  FP32: 64^3 9.5 + 9.5 us against 17 + 14 for the sweeps, 100^3 34 + 51
+// against 32 + 27.  FP64: 32^3 8.3 + 7.5 us against 16.5 + 10.6, 64^3 17.5 + 19.8
+// against 29 + 19.  An iteration of a whole solve with legs against one with
+// what runs above the line: FP32 64^3 90 and 112 us, 68^3 121.5 and 114.5, 76^3
+// 125 and 121; FP64 48^3 85 and 93, 52^3 114.5 and 106, 64^3 120 and 113; FP32
+// 8x180x180 392 and 471.  Levels with stored diagonals, which march in no
+// case, would gain a little beyond it (72^3 FP32 159 against 169 us, 64^3 FP64
+// 144 and 148) up to 84^3 (194 and 192; FP64 260 and 221); one line serves both.
 template <class T> constexpr long long kLegCells = sizeof(T) == 4 ? 300000 : 150000;
 template <class T>
 static bool leg_ok(const Level<T> &L, const Cycle &cy) {
@@ -2873,11 +2878,12 @@ static int leg_post(Level<T> &L, int l, const Level<T> &C, const T *b, const Cyc
 }
 
 // Whether level l's legs march (k_march): the default cycle on the larger
-// levels of a singular system.  256^3 FP32: 89 + 116 us against 198 + 162
-// for the sweeps and the restriction (FP64 164 + 206 against 484 + 409);
-// 128^3 FP32 23 + 25 against 42 + 38, FP64 36 + 30 against 82 + 54; 100^3
-// FP32 20 + 20 against 32 + 38.  64^3 FP64 16.5 + 15 against 17.5 + 21 for
-// the one-region legs; 64^3 FP32 15 + 13 against their 9.1 + 9.3.
+// levels of a singular system.  256^3 FP32: 105 + 121 us against 205 + 165
+// for the sweeps and the restriction (FP64 178 + 206 against 495 + 410);
+// 128^3 FP32 26 + 24.5 against 42.5 + 38, FP64 36.5 + 30.5 against 67 + 54;
+// 100^3 FP32 19.5 + 19 against 32 + 38 (26 and the CG sums' own pass).  64^3
+// FP64 18 + 16 against 17.5 + 21 for the one-region legs; 64^3 FP32 15 + 13
+// against their 9.5 + 9.5.
 template <class T>
 static bool march_ok(const Level<T> &L, const Cycle &cy) {
     return cy.fused && !cy.tri && cy.dgi && !cy.divide && cy.nu_pre == 2 && cy.nu_post == 2 && cy.rows == 0 && cy.planes == 0 &&

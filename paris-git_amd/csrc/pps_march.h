@@ -18,14 +18,16 @@
 // other's lines if they march at one pace.  So a block fills a CU: of two
 // 512-thread blocks (32 x 32 in FP32 too) one was served first and ran up to
 // 30 planes ahead, and its lines had gone when the other came: 389 and 534 MB
-// fetched at 256^3 (PRE, POST; least 268 and 310) instead of 332 and 429.
+// fetched at 256^3 (PRE, POST; least 268 and 310) instead of 337 and 423.
 //
 // Planes are loaded straight into LDS (buffer loads with an LDS target, two
 // planes ahead: no registers are held by loads in flight, and a load's
 // latency spans two steps).  Rows of one parity issue them at the start of a
 // step and the others at its end, so that half of the wavefronts compute
-// while the other half waits for the load unit (256^3 FP32 94 + 122 us with
-// all at the start, 89 + 116 so).  A thread owns the column of one x-pair (2m,
+// while the other half waits for the load unit (PRE + POST at 128^3 26.0 + 24.5
+// us, 27.4 + 26.7 with all at the start; FP64 36.5 + 30.5 against 38.9 + 35.2,
+// 256^3 FP64 178 + 206 against 181 + 209; 256^3 FP32 105 + 121 either way, 512^3
+// 785 + 882 against 777 + 872).  A thread owns the column of one x-pair (2m,
 // 2m+1) of one row: the rows of its last planes and all vertical neighbours
 // are in its registers, neighbours along x in the next lanes'; those along y
 // come from LDS, where each stage leaves the value it formed for the stage
@@ -258,7 +260,7 @@ k_march(LevelK<T> L, MarchK g, Coarsening cg, const T *__restrict__ b, const T *
     // until nothing older than what it and the step before issued since is
     // outstanding: its loads for plane s + 2 and both steps' stores, which
     // stay in flight (to wait for one of those loads costs a memory latency a
-    // step: 256^3 FP32 PRE 99 us, POST 135; counted 95 and 124).  A count too
+    // step: 256^3 FP32 PRE 111 us, POST 127; counted 105 and 121).  A count too
     // low is safe; one that takes in a store older than the loads waited for
     // is not, so a wavefront that requests at the start of a step must issue
     // those loads before the step's stores, which touch other memory: the

@@ -81,7 +81,8 @@ constexpr int kFoldParts = 128;
 // Of alpha's (k_update) and r.r's (the next cycle's first leg), one sum: up to
 // 1024, a load for each thread of a leg and four for one of k_update.  128^3:
 // k_update 12.9 -> 13.3 us without k_scal_alpha's 4.2, k_march PRE 23.3 ->
-// 23.5 without k_scal_rr's 4.6; solves at 128^3 1576 -> 1555 us, 64^3 FP64 873
+// 23.5 (means that take in a solve's last one, which returns at once) without
+// k_scal_rr's 4.6; solves at 128^3 1576 -> 1555 us, 64^3 FP64 873
 // -> 860, 49x64x40 FP64 1088 -> 1060.
 constexpr int kFoldWide = 1024;
 
